@@ -41,20 +41,29 @@ COUNTER_CMD = ("cd /tmp && export TMPDIR=/tmp && timeout -s KILL 90 rocprofv3 --
                "--no-cpu --prewarm 0 --ttr-seeds 0 --calibrate {mib}{extra}")
 
 
-def algorithmic_bytes(n, P, alg, recomputed_state=False):
+def support_rows(supp):
+    """Fraction of the rows that meet the support (an empty support counts every row)."""
+    hit = np.asarray(supp).reshape(-1, *np.shape(supp)[-2:]).astype(bool).any(axis=2).mean(axis=1)
+    return float(np.where(hit > 0, hit, 1.0).mean())
+
+
+def algorithmic_bytes(n, P, alg, recomputed_state=False, rows=1.0):
     """HBM bytes per launch of the two iteration kernels (algorithmic, no re-reads):
     column pass 16 B/px (+ the amplitude, 4 B/px once per launch); row update pass
     for HIO/RAAR 32.125 B/px with the state stored (the field read and written,
     rho_n read and written, the support as one bit per pixel) or 24.125 B/px with
     it recomputed from its row transform (the projected field and the state's row
-    transform read, the new row transform written, the support bits); ER 16.125
-    B/px in both forms."""
+    transform read, the new row transform written, the support bits), then of the
+    rows that meet the support (`rows`, their fraction) only; ER 16.125 B/px, with
+    the state recomputed of those rows only, the column pass too."""
     npx = n * n
     col = 16 * npx * P + 4 * npx
-    if alg in ("HIO", "RAAR"):
-        row = (24.125 if recomputed_state else 32.125) * npx * P
+    if recomputed_state:
+        if alg == "ER":
+            col = 16 * rows * npx * P + 4 * npx
+        row = (16.125 if alg == "ER" else 24.125) * rows * npx * P
     else:
-        row = 16.125 * npx * P
+        row = (16.125 if alg == "ER" else 32.125) * npx * P
     return col, row
 
 
@@ -134,7 +143,11 @@ def fused_flops(n, P, block):
     return 4 * (block + 1) * 5 * n * n * np.log2(n) * P
 
 
-def rocprof_kernel_name(kernel, n, alg, variant):
+def rocprof_kernel_name(kernel, n, alg, variant, recomputed=False):
+    if recomputed and kernel == "row":
+        return f"void spr::k_row_listed<{n}, {ROW_MODE[alg]}, {variant}>(spr::RowArgs, int)"
+    if recomputed and kernel == "col":
+        return f"void spr::k_col_step<{n}, {1 if alg == 'ER' else 0}, {variant}>(spr::StepArgs)"
     if kernel == "fused":
         return f"void spr::k_iter_fused<{n}, {ROW_MODE[alg]}>(spr::FusedArgs)"
     if kernel == "row":
@@ -424,10 +437,11 @@ def batch_bench(args, log):
     ind_iters = args.steps * args.batch_block * b.total
     value = ind_iters / dt
     # algorithmic bytes of one iteration of the whole batch: per individual 16
-    # B/px of column pass and 32.125 (state stored) or 24.125 (recomputed) of
-    # row pass, by the size class's row variant; each pattern's amplitude once
-    # per column pass
-    per_px = {n: 16 + (24.125 if hipcore.row_variant_recomputes_state(n, hipcore.default_variants(n)[1]) else 32.125)
+    # B/px of column pass and 32.125 (state stored) or 24.125 (recomputed, on the
+    # rows that meet the support) of row pass, by the size class's row variant;
+    # each pattern's amplitude once per column pass
+    per_px = {n: 16 + (24.125 * support_rows(starts[n][1])
+                       if hipcore.row_variant_recomputes_state(n, hipcore.default_variants(n)[1]) else 32.125)
               for n in set(sizes)}
     it_bytes = sum(per_px[n] * n * n * P + 4.0 * n * n for n in sizes)
     frac = it_bytes * (value / b.total) / 1e9 / HBM_PEAK_GBS
@@ -573,7 +587,8 @@ def main():
     chunk_bytes, chunk = be.chunk()
     fused = be.fused()[1]
     recomputed = hipcore.row_variant_recomputes_state(n, be.variants()[1])
-    col_b, row_b = algorithmic_bytes(n, min(P, chunk), args.alg, recomputed)   # per launch (one chunk)
+    rows = support_rows(be.get_population()[1])
+    col_b, row_b = algorithmic_bytes(n, min(P, chunk), args.alg, recomputed, rows)   # per launch (one chunk)
     iter_bytes = (col_b + row_b) / min(P, chunk)
     iteration_frac = value * iter_bytes / 1e9 / HBM_PEAK_GBS
     if not fused:
@@ -597,10 +612,10 @@ def main():
         # dominant kernel = the one with the larger share of the timed region
         cvar, rvar = be.variants()
         if row_ms >= col_ms:
-            dom = {"kernel": rocprof_kernel_name("row", n, args.alg, rvar), "achieved": row_gbs,
+            dom = {"kernel": rocprof_kernel_name("row", n, args.alg, rvar, recomputed), "achieved": row_gbs,
                    "bytes_per_launch": row_b, "avg_launch_us": row_avg * 1e6}
         else:
-            dom = {"kernel": rocprof_kernel_name("col", n, args.alg, cvar), "achieved": col_gbs,
+            dom = {"kernel": rocprof_kernel_name("col", n, args.alg, cvar, recomputed), "achieved": col_gbs,
                    "bytes_per_launch": col_b, "avg_launch_us": col_avg * 1e6}
         log(f"column pass: {col_cnt} launches, avg {col_avg * 1e6:.1f} us, {col_gbs:.0f} GB/s algorithmic")
         log(f"row pass:    {row_cnt} launches, avg {row_avg * 1e6:.1f} us, {row_gbs:.0f} GB/s algorithmic")

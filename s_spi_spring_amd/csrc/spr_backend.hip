@@ -56,6 +56,11 @@ struct spr_ctx {
     float2* work2 = nullptr;      // second half-transformed field per individual (correlations, |b|)
     uint8_t* supp = nullptr;
     uint32_t* sbits = nullptr;    // supports one bit per pixel, packed at the start of every iteration block
+    // Rows that meet each support, made with sbits (SupportPlan in spr_kernels.hpp).
+    int* rowcnt = nullptr;        // [cap]
+    uint16_t* rowlist = nullptr;  // [cap][n]
+    uint32_t* colmask = nullptr;  // [cap][n/V], V >= 8 values per thread of the column pass
+    uint32_t* rowflags = nullptr; // [cap][n/32]
     float* amp = nullptr;         // amplitudes [npat][n][n]
     float* amp_t = nullptr;       // amp transposed (read along columns by the column pass)
     int npat = 1;                 // patterns sharing this handle (one amplitude each)
@@ -177,12 +182,27 @@ PhaseCut cut_raar(float r) {
 template <int N, int RV> int launch_row_v(spr_ctx* c, int mode, const RowArgs& a, int cnt, hipStream_t s) {
     using G = typename RowVariant<N, RV>::G;
     const dim3 grid((unsigned)((size_t)cnt * N / G::RW)), block(G::ROW_THREADS);
+    if constexpr (G::ROW_RECOMPUTE) {
+        if (mode == ROW_HIO || mode == ROW_RAAR || mode == ROW_ER) {
+            if (mode == ROW_HIO) hipLaunchKernelGGL((k_row_listed<N, ROW_HIO, RV>), grid, block, 0, s, a, cnt);
+            else if (mode == ROW_RAAR) hipLaunchKernelGGL((k_row_listed<N, ROW_RAAR, RV>), grid, block, 0, s, a, cnt);
+            else hipLaunchKernelGGL((k_row_listed<N, ROW_ER, RV>), grid, block, 0, s, a, cnt);
+            SPR_HIP(c, hipGetLastError());
+            return SPR_OK;
+        }
+    }
     switch (mode) {
         case ROW_FWD: hipLaunchKernelGGL((k_row<N, ROW_FWD, RV>), grid, block, 0, s, a); break;
         case ROW_FINAL: hipLaunchKernelGGL((k_row<N, ROW_FINAL, RV>), grid, block, 0, s, a); break;
-        case ROW_HIO: hipLaunchKernelGGL((k_row<N, ROW_HIO, RV>), grid, block, 0, s, a); break;
-        case ROW_RAAR: hipLaunchKernelGGL((k_row<N, ROW_RAAR, RV>), grid, block, 0, s, a); break;
-        case ROW_ER: hipLaunchKernelGGL((k_row<N, ROW_ER, RV>), grid, block, 0, s, a); break;
+        case ROW_HIO:
+            if constexpr (!G::ROW_RECOMPUTE) hipLaunchKernelGGL((k_row<N, ROW_HIO, RV>), grid, block, 0, s, a);
+            break;
+        case ROW_RAAR:
+            if constexpr (!G::ROW_RECOMPUTE) hipLaunchKernelGGL((k_row<N, ROW_RAAR, RV>), grid, block, 0, s, a);
+            break;
+        case ROW_ER:
+            if constexpr (!G::ROW_RECOMPUTE) hipLaunchKernelGGL((k_row<N, ROW_ER, RV>), grid, block, 0, s, a);
+            break;
         case ROW_FWD_INPLACE: hipLaunchKernelGGL((k_row<N, ROW_FWD_INPLACE, RV>), grid, block, 0, s, a); break;
         case ROW_INV_INPLACE: hipLaunchKernelGGL((k_row<N, ROW_INV_INPLACE, RV>), grid, block, 0, s, a); break;
         default: return fail(c, SPR_ERR_ARG, "bad row mode");
@@ -220,12 +240,21 @@ template <int N> int launch_row(spr_ctx* c, int mode, const RowArgs& a, int cnt,
 
 // Column passes: the projection pass in every variant, the plain transforms
 // (2-D FT / IFT, off the iteration path) in variant 0; in place, or into `out`.
+// Whether a row variant of size N recomputes the state.
+template <int N, int RV = 0> constexpr bool has_recompute() {
+    if constexpr (RV < MAX_VARIANTS) {
+        if constexpr (RowVariant<N, RV>::valid)
+            if (RowVariant<N, RV>::G::ROW_RECOMPUTE) return true;
+        return has_recompute<N, RV + 1>();
+    }
+    return false;
+}
 template <int N, int CV>
-int launch_col_v(spr_ctx* c, int mode, float2* f, int cnt, hipStream_t s, int first, float2* out = nullptr) {
+int launch_col_v(spr_ctx* c, int mode, float2* f, int cnt, hipStream_t s, int first) {
     using G = typename ColVariant<N, CV>::G;
     if (G::TW_GLOBAL && !c->twtab[CV]) return fail(c, SPR_ERR_STATE, "twiddle table missing");
-    const ColArgs a{f, c->amp, c->tw, c->amp_t, c->amp_of ? c->amp_of + first : nullptr, c->twtab[CV], out ? out : f};
-    const dim3 grid((unsigned)((size_t)cnt * (N / G::COL_STRIP))), block(G::COL_THREADS);
+    const ColArgs a{f, c->amp, c->tw, c->amp_t, c->amp_of ? c->amp_of + first : nullptr, c->twtab[CV], f};
+    const dim3 grid((unsigned)((size_t)cnt * (N / G::C))), block(G::COL_THREADS);
     switch (mode) {
         case COL_PROJ: hipLaunchKernelGGL((k_col<N, COL_PROJ, CV>), grid, block, 0, s, a); break;
         case COL_FWD:
@@ -240,51 +269,74 @@ int launch_col_v(spr_ctx* c, int mode, float2* f, int cnt, hipStream_t s, int fi
     return SPR_OK;
 }
 
-// Global twiddle tables of every column variant of size N that reads one.
+// The projection pass over individuals [first, first + cnt) of an iteration that
+// recomputes rho_n (StepArgs), f and proj at the first of them.
+struct Step {
+    int mode;
+    float2 *f, *proj;
+    float lin_w, lin_p;
+    int all_rows;
+};
+template <int N, int CV> int launch_step_v(spr_ctx* c, const Step& st, int cnt, hipStream_t s, int first) {
+    if constexpr (has_recompute<N>()) {
+        using G = typename ColVariant<N, CV>::G;
+        if (!c->twtab[CV]) return fail(c, SPR_ERR_STATE, "twiddle table missing");
+        const StepArgs a{st.f, st.proj, c->amp, c->amp_of ? c->amp_of + first : nullptr, c->twtab[CV],
+                         c->colmask + (size_t)first * G::T, st.lin_w, st.lin_p, st.all_rows};
+        const dim3 grid((unsigned)((size_t)cnt * (N / G::C))), block(G::COL_THREADS);
+        switch (st.mode) {
+            case STEP_LIN: hipLaunchKernelGGL((k_col_step<N, STEP_LIN, CV>), grid, block, 0, s, a); break;
+            case STEP_ER: hipLaunchKernelGGL((k_col_step<N, STEP_ER, CV>), grid, block, 0, s, a); break;
+            case STEP_ER_LAST: hipLaunchKernelGGL((k_col_step<N, STEP_ER_LAST, CV>), grid, block, 0, s, a); break;
+            default: return fail(c, SPR_ERR_ARG, "bad step mode");
+        }
+        SPR_HIP(c, hipGetLastError());
+        return SPR_OK;
+    } else {
+        return fail(c, SPR_ERR_ARG, "no iteration with a recomputed state for this grid size");
+    }
+}
+template <int N, int CV = 0> int launch_step(spr_ctx* c, const Step& st, int cnt, hipStream_t s, int first) {
+    if constexpr (CV < MAX_VARIANTS) {
+        if constexpr (ColVariant<N, CV>::valid) {
+            if (c->colvar == CV) {
+                constexpr int CN = narrow_variant<N, CV>();
+                if (CN != CV && cnt * (N / ColVariant<N, CV>::G::C) < 256) return launch_step_v<N, CN>(c, st, cnt, s, first);
+                return launch_step_v<N, CV>(c, st, cnt, s, first);
+            }
+        }
+        return launch_step<N, CV + 1>(c, st, cnt, s, first);
+    } else {
+        return fail(c, SPR_ERR_ARG, "bad column variant");
+    }
+}
+
+// Global twiddle tables of every column variant of size N (read by the step
+// passes, and by the column passes of variants with TW_GLOBAL).
 template <int N, int CV = 0> int build_twtabs(spr_ctx* c) {
     if constexpr (CV < MAX_VARIANTS) {
         if constexpr (ColVariant<N, CV>::valid) {
             using G = typename ColVariant<N, CV>::G;
-            if constexpr (G::TW_GLOBAL) {
-                constexpr int SIZE = TwTableP<typename G::PL>::SIZE;
-                SPR_HIP(c, hipMalloc(&c->twtab[CV], SIZE * sizeof(float2)));
-                hipLaunchKernelGGL((k_build_twtab<typename G::PL>), dim3(1), dim3(256), 0, c->stream, c->twtab[CV],
-                                   (const float2*)c->tw);
-                SPR_HIP(c, hipGetLastError());
-            }
+            constexpr int SIZE = TwTableP<typename G::PL>::SIZE;
+            SPR_HIP(c, hipMalloc(&c->twtab[CV], SIZE * sizeof(float2)));
+            hipLaunchKernelGGL((k_build_twtab<typename G::PL>), dim3(1), dim3(256), 0, c->stream, c->twtab[CV],
+                               (const float2*)c->tw);
+            SPR_HIP(c, hipGetLastError());
         }
         return build_twtabs<N, CV + 1>(c);
     }
     return SPR_OK;
 }
 
-template <int N> int launch_col(spr_ctx* c, int mode, float2* f, int cnt, hipStream_t s, int first, float2* out) {
-    if (mode != COL_PROJ) return launch_col_v<N, 0>(c, mode, f, cnt, s, first, out);
-    switch (c->colvar) {
-        case 0: return launch_col_v<N, 0>(c, mode, f, cnt, s, first, out);
-        case 1:
-            if constexpr (ColVariant<N, 1>::valid) return launch_col_v<N, 1>(c, mode, f, cnt, s, first, out);
-            break;
-        case 2:
-            if constexpr (ColVariant<N, 2>::valid) return launch_col_v<N, 2>(c, mode, f, cnt, s, first, out);
-            break;
-        case 3:
-            if constexpr (ColVariant<N, 3>::valid) return launch_col_v<N, 3>(c, mode, f, cnt, s, first, out);
-            break;
-        case 4:
-            if constexpr (ColVariant<N, 4>::valid) return launch_col_v<N, 4>(c, mode, f, cnt, s, first, out);
-            break;
-        case 5:
-            if constexpr (ColVariant<N, 5>::valid) return launch_col_v<N, 5>(c, mode, f, cnt, s, first, out);
-            break;
-        case 6:
-            if constexpr (ColVariant<N, 6>::valid) return launch_col_v<N, 6>(c, mode, f, cnt, s, first, out);
-            break;
-        case 7:
-            if constexpr (ColVariant<N, 7>::valid) return launch_col_v<N, 7>(c, mode, f, cnt, s, first, out);
-            break;
+template <int N, int CV = 0> int launch_col(spr_ctx* c, int mode, float2* f, int cnt, hipStream_t s, int first) {
+    if (mode != COL_PROJ) return launch_col_v<N, 0>(c, mode, f, cnt, s, first);
+    if constexpr (CV < MAX_VARIANTS) {
+        if constexpr (ColVariant<N, CV>::valid)
+            if (c->colvar == CV) return launch_col_v<N, plain_variant<N, CV>()>(c, mode, f, cnt, s, first);
+        return launch_col<N, CV + 1>(c, mode, f, cnt, s, first);
+    } else {
+        return fail(c, SPR_ERR_ARG, "bad column variant");
     }
-    return fail(c, SPR_ERR_ARG, "bad column variant");
 }
 
 // Grid sizes with compiled kernels (RadixPlan in spr_fft.hpp).
@@ -306,10 +358,12 @@ template <int N> int launch_col(spr_ctx* c, int mode, float2* f, int cnt, hipStr
 int row_n(spr_ctx* c, int mode, const RowArgs& a, int cnt, hipStream_t s) {
     SPR_DISPATCH_N(c, launch_row, c, mode, a, cnt, s);
 }
-// Column pass over fields f[0, cnt), the individuals [first, first + cnt),
-// in place or into out[0, cnt).
-int col_n(spr_ctx* c, int mode, float2* f, int cnt, hipStream_t s, int first = 0, float2* out = nullptr) {
-    SPR_DISPATCH_N(c, launch_col, c, mode, f, cnt, s, first, out);
+// Column pass over fields f[0, cnt), the individuals [first, first + cnt), in place.
+int col_n(spr_ctx* c, int mode, float2* f, int cnt, hipStream_t s, int first = 0) {
+    SPR_DISPATCH_N(c, launch_col, c, mode, f, cnt, s, first);
+}
+int step_n(spr_ctx* c, const Step& st, int cnt, hipStream_t s, int first) {
+    SPR_DISPATCH_N(c, launch_step, c, st, cnt, s, first);
 }
 
 // Timed passes (spr_timing) over `cnt` individuals from the argument pointers
@@ -322,15 +376,14 @@ int row(spr_ctx* c, int mode, const RowArgs& a, int cnt = -1) {
     if (rc != SPR_OK) return rc;
     return timing_end(c);
 }
-int col(spr_ctx* c, int mode, float2* f, int cnt = -1, int first = 0, float2* out = nullptr) {
+int col(spr_ctx* c, int mode, float2* f, int cnt = -1, int first = 0) {
     const int kind = (mode == COL_PROJ) ? SPR_KIND_COL_PROJ : SPR_KIND_COL_OTHER;
     int rc = timing_begin(c, kind);
     if (rc != SPR_OK) return rc;
-    rc = col_n(c, mode, f, cnt < 0 ? c->P : cnt, c->stream, first, out);
+    rc = col_n(c, mode, f, cnt < 0 ? c->P : cnt, c->stream, first);
     if (rc != SPR_OK) return rc;
     return timing_end(c);
 }
-
 RowArgs row_args(spr_ctx* c) {
     RowArgs a{};
     a.rho = c->rho;
@@ -341,8 +394,10 @@ RowArgs row_args(spr_ctx* c) {
     a.beta = 0.f;
     a.inv_nn = 1.0f / (float)((double)c->n * c->n);
     a.pc = cut_er_hio(0.f);
-    a.proj = nullptr;
+    a.proj = c->work2;
     a.inv_n = 1.0f / (float)c->n;
+    a.rowcnt = c->rowcnt;
+    a.rowlist = c->rowlist;
     return a;
 }
 
@@ -600,15 +655,49 @@ float key_value(unsigned long long k) {
 }
 int key_index(unsigned long long k) { return k ? (int)(0xFFFFFFFFu - (unsigned)(k & 0xFFFFFFFFu)) : 0; }
 
-// supp -> sbits for individuals [0, cnt) from the pointers given (one bit per
-// pixel, read by the row update passes).
-int pack_support(spr_ctx* c, const uint8_t* supp, uint32_t* bits, int cnt, hipStream_t s) {
-    const size_t nwords = (size_t)cnt * c->n * c->n / 32;
-    if (nwords == 0) return SPR_OK;
-    const dim3 grid((unsigned)std::min<size_t>((nwords + 255) / 256, 8192));
-    hipLaunchKernelGGL(k_pack_support, grid, dim3(256), 0, s, supp, bits, nwords);
+// Threads per line of column variant cv of size N.
+template <int N, int CV = 0> int col_lines_n(int cv) {
+    if constexpr (CV < MAX_VARIANTS) {
+        if constexpr (ColVariant<N, CV>::valid)
+            if (cv == CV) return ColVariant<N, CV>::G::T;
+        return col_lines_n<N, CV + 1>(cv);
+    }
+    return 0;
+}
+int col_lines(int n, int cv) {
+#define SPR_LINES_CASE(N_) if (n == N_) return col_lines_n<N_>(cv);
+    SPR_SIZES(SPR_LINES_CASE)
+#undef SPR_LINES_CASE
+    return 0;
+}
+
+// The support bits, row lists and column masks of all resident individuals, for
+// the handle's current column variant.
+int pack_support(spr_ctx* c, hipStream_t s) {
+    if (c->P <= 0) return SPR_OK;
+    const SupportPlan a{c->supp, c->sbits, c->rowcnt, c->rowlist, c->colmask, c->rowflags, c->n,
+                        col_lines(c->n, c->colvar)};
+    hipLaunchKernelGGL(k_pack_support, dim3((unsigned)(c->n / 32 * c->P)), dim3(256), 0, s, a);
+    SPR_HIP(c, hipGetLastError());
+    if (!row_recomputes(c->n, c->rowvar)) return SPR_OK;
+    hipLaunchKernelGGL(k_row_plan, dim3((unsigned)c->P), dim3(256), 0, s, a);
     SPR_HIP(c, hipGetLastError());
     return SPR_OK;
+}
+
+// The projection pass of iteration i of a block (i = niter: the trailing one) over
+// individuals [first, first + cnt), whose fields `a` points to.
+int project(spr_ctx* c, int row_mode, const RowArgs& a, bool rs, int i, int niter, int cnt, hipStream_t s, int first) {
+    if (!rs || (i == niter && row_mode != ROW_ER)) return col_n(c, COL_PROJ, a.work, cnt, s, first);
+    Step st{STEP_LIN, a.work, const_cast<float2*>(a.proj), 1.f, -(a.beta * a.inv_n), 0};
+    if (row_mode == ROW_RAAR) {
+        st.lin_w = a.beta;
+        st.lin_p = (1.f - 2.f * a.beta) * a.inv_n;
+    } else if (row_mode == ROW_ER) {
+        st.mode = i == niter ? STEP_ER_LAST : STEP_ER;
+        st.all_rows = i == 0;
+    }
+    return step_n(c, st, cnt, s, first);
 }
 
 // Pipelined form of the iteration over two halves of the population: lane 1
@@ -620,34 +709,28 @@ int pack_support(spr_ctx* c, const uint8_t* supp, uint32_t* bits, int cnt, hipSt
 int queue_iterate_lanes(spr_ctx* c, int mode, int niter, const RowArgs& a0) {
     const int h = (c->P + 1) / 2, h2 = c->P - h;
     const size_t off = (size_t)h * c->n * c->n;
-    // With a row variant that recomputes rho_n the column passes project into work2.
     const bool rs = row_recomputes(c->n, c->rowvar);
-    float2* pa = rs ? c->work2 : nullptr;
-    float2* pb = rs ? c->work2 + off : nullptr;
-    RowArgs a = a0;
-    a.proj = pa;
+    const RowArgs a = a0;
     RowArgs b = a;
     b.rho += off;
     b.work += off;
     b.supp += off;
     b.sbits += off / 32;
-    b.proj = pb;
+    b.rowcnt += h;
+    b.rowlist += (size_t)h * c->n;
+    b.proj += off;
     hipStream_t s1 = c->stream, s2 = c->lane2;
-    SPR_TRY(pack_support(c, c->supp, c->sbits, c->P, s1));
+    SPR_TRY(pack_support(c, s1));
     SPR_TRY(row_n(c, ROW_FWD, a, h, s1));
     SPR_HIP(c, hipEventRecord(c->ev_fork, s1));
     SPR_HIP(c, hipStreamWaitEvent(s2, c->ev_fork, 0));
     SPR_TRY(row_n(c, ROW_FWD, b, h2, s2));
-    for (int i = 0; i < niter; ++i) {
-        SPR_TRY(col_n(c, COL_PROJ, a.work, h, s1, 0, pa));
-        SPR_TRY(col_n(c, COL_PROJ, b.work, h2, s2, h, pb));
-        SPR_TRY(row_n(c, mode, a, h, s1));
-        SPR_TRY(row_n(c, mode, b, h2, s2));
+    for (int i = 0; i <= niter; ++i) {
+        SPR_TRY(project(c, mode, a, rs, i, niter, h, s1, 0));
+        SPR_TRY(project(c, mode, b, rs, i, niter, h2, s2, h));
+        SPR_TRY(row_n(c, i < niter ? mode : ROW_FINAL, a, h, s1));
+        SPR_TRY(row_n(c, i < niter ? mode : ROW_FINAL, b, h2, s2));
     }
-    SPR_TRY(col_n(c, COL_PROJ, a.work, h, s1, 0, pa));
-    SPR_TRY(col_n(c, COL_PROJ, b.work, h2, s2, h, pb));
-    SPR_TRY(row_n(c, ROW_FINAL, a, h, s1));
-    SPR_TRY(row_n(c, ROW_FINAL, b, h2, s2));
     SPR_HIP(c, hipEventRecord(c->ev_join, s2));
     SPR_HIP(c, hipStreamWaitEvent(s1, c->ev_join, 0));
     return SPR_OK;
@@ -678,7 +761,7 @@ int queue_iterate_block(spr_ctx* c, int mode, int niter, const RowArgs& a0) {
     const int chunk = chunk_individuals(c);
     const size_t np = (size_t)c->n * c->n;
     const bool rs = row_recomputes(c->n, c->rowvar);
-    SPR_TRY(pack_support(c, a0.supp, const_cast<uint32_t*>(a0.sbits), c->P, c->stream));
+    SPR_TRY(pack_support(c, c->stream));
     for (int first = 0; first < c->P; first += chunk) {
         const int cnt = std::min(chunk, c->P - first);
         RowArgs a = a0;
@@ -686,15 +769,16 @@ int queue_iterate_block(spr_ctx* c, int mode, int niter, const RowArgs& a0) {
         a.work += first * np;
         a.supp += first * np;
         a.sbits += first * np / 32;
-        float2* pj = rs ? c->work2 + first * np : nullptr;
-        a.proj = pj;
+        a.rowcnt += first;
+        a.rowlist += (size_t)first * c->n;
+        a.proj += first * np;
         SPR_TRY(row(c, ROW_FWD, a, cnt));
-        for (int i = 0; i < niter; ++i) {
-            SPR_TRY(col(c, COL_PROJ, a.work, cnt, first, pj));
-            SPR_TRY(row(c, mode, a, cnt));
+        for (int i = 0; i <= niter; ++i) {
+            SPR_TRY(timing_begin(c, SPR_KIND_COL_PROJ));
+            SPR_TRY(project(c, mode, a, rs, i, niter, cnt, c->stream, first));
+            SPR_TRY(timing_end(c));
+            SPR_TRY(row(c, i < niter ? mode : ROW_FINAL, a, cnt));
         }
-        SPR_TRY(col(c, COL_PROJ, a.work, cnt, first, pj));
-        SPR_TRY(row(c, ROW_FINAL, a, cnt));
     }
     return SPR_OK;
 }
@@ -857,7 +941,7 @@ template <int N, int CV> int launch_col_loss_v(spr_ctx* c, LossArgs a, int items
     using G = typename ColVariant<N, CV>::G;
     if (G::TW_GLOBAL && !c->twtab[CV]) return fail(c, SPR_ERR_STATE, "twiddle table missing");
     a.twtab = c->twtab[CV];
-    const dim3 grid((unsigned)((size_t)items * (N / G::COL_STRIP))), block(G::COL_THREADS);
+    const dim3 grid((unsigned)((size_t)items * (N / G::C))), block(G::COL_THREADS);
     if (want_loss) hipLaunchKernelGGL((k_col_loss<N, CV, true>), grid, block, 0, c->stream, a);
     else hipLaunchKernelGGL((k_col_loss<N, CV, false>), grid, block, 0, c->stream, a);
     SPR_HIP(c, hipGetLastError());
@@ -869,7 +953,7 @@ template <int N, int CV> int launch_col_loss_v(spr_ctx* c, LossArgs a, int items
 template <int N, int CV> constexpr bool same_plan_variant() {
     if constexpr (ColVariant<N, CV>::valid) {
         using G = typename ColVariant<N, CV>::G;
-        return G::COL_GROUPS == 1 && !G::COL_WAVE && std::is_same<typename G::PL, RadixPlan<N>>::value;
+        return !G::COL_WAVE && std::is_same<typename G::PL, RadixPlan<N>>::value;
     }
     return false;
 }
@@ -1079,11 +1163,10 @@ VariantPair default_variants(int n) {
 // its column passes project into work2.
 int time_iteration(spr_ctx* c, const RowArgs& ra0, int reps, hipEvent_t e0, hipEvent_t e1, float* ms) {
     RowArgs ra = ra0;
-    float2* out = nullptr;
-    if (row_recomputes(c->n, c->rowvar)) {
-        ra.proj = c->work2;
-        out = c->work2;
-    } else {
+    const bool rs = row_recomputes(c->n, c->rowvar);
+    SPR_TRY(pack_support(c, c->stream));   // the column masks follow the column variant
+    SPR_TRY(row_n(c, ROW_FWD, ra, c->P, c->stream));
+    if (!rs) {
         const int np = c->n * c->n;
         hipLaunchKernelGGL(k_copy_fields, dim3((np + 255) / 256, c->P), dim3(256), 0, c->stream, (const float2*)c->rho,
                            (const int*)nullptr, c->work2, (const int*)nullptr, np);
@@ -1091,7 +1174,7 @@ int time_iteration(spr_ctx* c, const RowArgs& ra0, int reps, hipEvent_t e0, hipE
         ra.rho = c->work2;
     }
     auto once = [&]() {
-        SPR_TRY(col_n(c, COL_PROJ, c->work, c->P, c->stream, 0, out));
+        SPR_TRY(project(c, ROW_RAAR, ra, rs, 0, 1, c->P, c->stream, 0));
         return row_n(c, ROW_RAAR, ra, c->P, c->stream);
     };
     SPR_TRY(once());   // warm-up (code load, caches)
@@ -1122,8 +1205,6 @@ int autotune(spr_ctx* c, int reps, float* col_ms, float* row_ms) {
     ra.pc = cut_raar(0.f);
     const VariantPair keep{c->colvar, c->rowvar};
     c->rowvar = 0;
-    SPR_TRY(row_n(c, ROW_FWD, ra, c->P, c->stream));   // realistic spectra in work
-    SPR_TRY(pack_support(c, c->supp, c->sbits, c->P, c->stream));
     hipEvent_t e0 = nullptr, e1 = nullptr;
     SPR_HIP(c, hipEventCreate(&e0));
     if (hipEventCreate(&e1) != hipSuccess) {
@@ -1335,6 +1416,11 @@ static int create_context(spr_ctx** out, int n, int capacity, int npat, const fl
         return cleanup_fail("hipMalloc work", e);
     if ((e = hipMalloc(&c->supp, np * capacity)) != hipSuccess) return cleanup_fail("hipMalloc supp", e);
     if ((e = hipMalloc(&c->sbits, np / 8 * capacity)) != hipSuccess) return cleanup_fail("hipMalloc sbits", e);
+    if ((e = hipMalloc(&c->rowcnt, (size_t)capacity * sizeof(int))) != hipSuccess ||
+        (e = hipMalloc(&c->rowlist, (size_t)capacity * n * sizeof(uint16_t))) != hipSuccess ||
+        (e = hipMalloc(&c->colmask, (size_t)capacity * (n / 8) * sizeof(uint32_t))) != hipSuccess ||
+        (e = hipMalloc(&c->rowflags, (size_t)capacity * (n / 32) * sizeof(uint32_t))) != hipSuccess)
+        return cleanup_fail("hipMalloc row lists", e);
     if ((e = hipMalloc(&c->amp, np * npat * sizeof(float))) != hipSuccess) return cleanup_fail("hipMalloc amp", e);
     if ((e = hipMalloc(&c->amp_t, np * npat * sizeof(float))) != hipSuccess) return cleanup_fail("hipMalloc amp_t", e);
     if ((e = hipMalloc(&c->tw, n * sizeof(float2))) != hipSuccess) return cleanup_fail("hipMalloc tw", e);
@@ -1409,6 +1495,10 @@ int spr_destroy(spr_ctx* c) {
     (void)hipFree(c->work);
     (void)hipFree(c->supp);
     (void)hipFree(c->sbits);
+    (void)hipFree(c->rowcnt);
+    (void)hipFree(c->rowlist);
+    (void)hipFree(c->colmask);
+    (void)hipFree(c->rowflags);
     (void)hipFree(c->amp);
     (void)hipFree(c->amp_t);
     (void)hipFree(c->amp_of);

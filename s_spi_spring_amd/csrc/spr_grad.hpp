@@ -37,8 +37,8 @@ __global__ __launch_bounds__((ColVariant<N, CV>::G::COL_THREADS))
 __attribute__((amdgpu_waves_per_eu((ColVariant<N, CV>::G::COL_WAVES_PER_EU)))) void k_col_loss(LossArgs a) {
     using G = typename ColVariant<N, CV>::G;
     using PL = typename G::PL;
-    constexpr int V = G::V, T = G::T, C = G::C, NT = G::COL_THREADS, TILES = N / G::COL_STRIP;
-    static_assert(G::COL_GROUPS == 1 && !G::COL_WAVE, "loss passes use single-group LDS tiles");
+    constexpr int V = G::V, T = G::T, C = G::C, NT = G::COL_THREADS, TILES = N / C;
+    static_assert(!G::COL_WAVE, "loss passes use LDS tiles of rows");
     __shared__ float2 twl[G::TW_GLOBAL ? 1 : TwTableP<PL>::SIZE];
     __shared__ float2 lds[G::COL_TILE];
     __shared__ double red[WANT_LOSS ? 4 * (NT / 64) : 1];
@@ -46,7 +46,7 @@ __attribute__((amdgpu_waves_per_eu((ColVariant<N, CV>::G::COL_WAVES_PER_EU)))) v
     const float2* tw = twl;
     if constexpr (G::TW_GLOBAL) tw = a.twtab;
     else tw_fill_p<PL>(twl, a.tw, tid, NT);
-    const int strip = col_strip<N, G::COL_STRIP>(blockIdx.x);
+    const int strip = col_strip<N, C>(blockIdx.x);
     const int item = strip / TILES;
     const int x0 = (strip % TILES) * C;
     float2* __restrict__ f = a.f + (size_t)item * N * N + x0;

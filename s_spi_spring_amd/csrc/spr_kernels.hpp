@@ -18,14 +18,16 @@
 //     row pass     rho' = rowIFFT(work)/N^2 ; rho <- update(rho', rho, S) ;
 //                  work <- rowFFT(rho)                                32.125 B/px
 //   state recomputed (work holds rowFFT(rho_n); rho is read and written only at
-//   the ends of a block)
-//     column pass  proj <- colIFFT( P_M( colFFT(work) ) )                   16 B/px
-//     row pass     HIO: rho' = rowIFFT(proj)/N^2 ; rho_n = rowIFFT(work)/N ;
+//   the ends of a block), with h the fraction of the rows that meet the support
+//     column pass  proj <- colIFFT( P_M( colFFT(work) ) ) on those rows; on the
+//                  others the update, linear there, in place in work    16 B/px
+//     row pass     on those rows only:
+//                  HIO: rho' = rowIFFT(proj)/N^2 ; rho_n = rowIFFT(work)/N ;
 //                       work <- rowFFT(update(rho', rho_n, S))
 //                  RAAR: q = rowIFFT(2 proj/N^2 - work/N) (= 2 rho' - rho_n) ;
 //                       work <- proj/N - beta rowFFT(q on the rejected pixels)
-//                                                                     24.125 B/px
-// so HIO/RAAR move 48.125 or 40.125 B/px per individual-iteration (the second
+//                                                                 24.125 h B/px
+// so HIO/RAAR move 48.125 or 16 + 24.125 h B/px per individual-iteration (the second
 // form saves the state's round trip for one more row transform in HIO and none
 // in RAAR); ER, which needs no rho_n, moves 32.125 B/px in both. proj is the
 // work2 buffer. (The support packing reads 1 and writes 0.125 B/px once per
@@ -52,15 +54,12 @@ constexpr int pow2_floor(int x) { return x >= 2 ? 2 * pow2_floor(x / 2) : 1; }
 // pass's twiddle table from global memory (through the caches) instead of
 // building it in LDS. CSK > 0 lays the column tile out unpadded with one spare
 // tile row after every 2^CSK rows (row i of the tile at (i + i/2^CSK) * C; PAD
-// is then unused). CGR > 1 gives each column-pass workgroup CGR adjacent groups
-// of C columns (a strip of C*CGR columns, so that C*CGR = 16 reads whole
-// 128-byte row segments), transformed one group after another through the same
-// C-column LDS tile; WPE > 0 sets the column pass's waves per SIMD (its
-// register budget) instead of deriving it from the workgroups a CU holds.
+// is then unused). WPE > 0 sets the column pass's waves per SIMD (its register
+// budget) instead of deriving it from the workgroups a CU holds.
 // RST = 1 makes the row update passes recompute rho_n from its row transform
 // instead of reading and writing it (the second iteration form above).
 template <int N, class PL_ = RadixPlan<N>, int CCOLS = 0, int RTHREADS = 256, int RPF = -1, int PAD = 1, int TWG = 0,
-          int RSH = 3, int CSK = 0, int CGR = 1, int WPE = 0, int RST = 0>
+          int RSH = 3, int CSK = 0, int WPE = 0, int RST = 0>
 struct GeoT {
     using PL = PL_;
     static constexpr bool TW_GLOBAL = TWG != 0;
@@ -86,8 +85,6 @@ struct GeoT {
 #endif
     // columns per column-pass workgroup: a power of two (it divides N)
     static constexpr int C = CCOLS ? CCOLS : (pow2_floor(SPR_COL_COLUMNS / N) < N ? pow2_floor(SPR_COL_COLUMNS / N) : N);
-    static constexpr int COL_GROUPS = CGR;                // groups of C columns per column-pass workgroup
-    static constexpr int COL_STRIP = C * CGR;             // columns per column-pass workgroup
     static constexpr bool COL_WAVE = SPR_COL_WAVE && T <= 64;
     static constexpr int COL_THREADS = C * T;
     static constexpr int CS = C + PAD;                    // padded LDS row length of a column tile
@@ -114,8 +111,7 @@ struct GeoT {
                                                             : (COL_WG_SLOTS < SPR_COL_WG_PER_CU ? COL_WG_SLOTS : SPR_COL_WG_PER_CU);
     static constexpr int COL_WAVES_PER_EU = WPE > 0 ? WPE : (COL_WG > 0 ? COL_WG : 1) * COL_THREADS / 256;
     static_assert(RW >= 1 && ROW_THREADS % T == 0 && N % RW == 0, "row geometry");
-    static_assert(COL_THREADS <= 1024 && N % COL_STRIP == 0, "column geometry");
-    static_assert(CGR == 1 || !COL_WAVE, "column groups need the tile layout");
+    static_assert(COL_THREADS <= 1024 && N % C == 0, "column geometry");
 };
 template <int N> using Geo = GeoT<N>;
 
@@ -136,43 +132,42 @@ template <int N> struct RowVariant<N, 0> { static constexpr bool valid = true; u
 // column variants: plan, columns per workgroup
 SPR_COL_VARIANT(256, 1, RadixPlan<256>, 16)
 SPR_COL_VARIANT(256, 2, RadixPlan<256>, 8)
+SPR_COL_VARIANT(256, 3, Plan<256, 16, 16, 16>, 16, 256, -1, 1, 0, 3, 0, 4)
+SPR_COL_VARIANT(256, 4, Plan<256, 16, 16, 16>, 8, 256, -1, 1, 0, 3, 0, 4)
 SPR_COL_VARIANT(384, 1, RadixPlan<384>, 8)
 SPR_COL_VARIANT(384, 2, RadixPlan<384>, 32)
 SPR_COL_VARIANT(384, 3, RadixPlan<384>, 4)
 SPR_COL_VARIANT(512, 1, RadixPlan<512>, 8)
 SPR_COL_VARIANT(512, 2, Plan<512, 16, 16, 4, 8>, 16)
 SPR_COL_VARIANT(512, 3, RadixPlan<512>, 4)
-SPR_COL_VARIANT(768, 1, RadixPlan<768>, 4, 256, -1, 1, 0, 3, 0, 4, 2)   // 4 groups of 4 columns
 SPR_COL_VARIANT(768, 2, RadixPlan<768>, 4)
-SPR_COL_VARIANT(1024, 1, Plan<1024, 16, 16, 8, 8>, 8, 256, -1, 1, 1, 3, 0, 2, 4)   // 2 groups of 8
 SPR_COL_VARIANT(1024, 2, Plan<1024, 16, 16, 8, 8>, 8)
-SPR_COL_VARIANT(1024, 3, Plan<1024, 16, 16, 8, 8>, 8, 256, -1, 0, 1, 3, 0, 2, 4)   // 2 groups of 8, unpadded
 SPR_COL_VARIANT(1024, 4, Plan<1024, 16, 16, 8, 8>, 8, 256, -1, 0, 0, 3, 4)
-// (plan, columns, -, -, padding, global twiddles): tiles under 80 KB, two workgroups per CU
+// (plan, columns, -, -, padding, global twiddles, -, -, waves per SIMD): tiles
+// under 80 KB, two workgroups per CU
 SPR_COL_VARIANT(384, 4, RadixPlan<384>, 16, 256, -1, 1, 1)
 SPR_COL_VARIANT(512, 4, RadixPlan<512>, 16, 256, -1, 1, 1)
 SPR_COL_VARIANT(512, 5, RadixPlan<512>, 8, 256, -1, 1, 1)
 SPR_COL_VARIANT(768, 3, RadixPlan<768>, 8, 256, -1, 1, 1)
 SPR_COL_VARIANT(768, 4, RadixPlan<768>, 8, 256, -1, 0, 1)
 SPR_COL_VARIANT(768, 5, RadixPlan<768>, 4, 256, -1, 1, 1)
+SPR_COL_VARIANT(768, 7, RadixPlan<768>, 8, 256, -1, 0, 1, 3, 0, 4)
+SPR_COL_VARIANT(1024, 1, Plan<1024, 16, 16, 8, 8>, 8, 256, -1, 1, 1, 3, 0, 4)
+SPR_COL_VARIANT(1024, 3, Plan<1024, 16, 16, 8, 8>, 8, 256, -1, 0, 1, 3, 0, 4)
 SPR_COL_VARIANT(1024, 5, Plan<1024, 16, 16, 8, 8>, 8, 256, -1, 1, 1)
 SPR_COL_VARIANT(1024, 6, Plan<1024, 16, 16, 8, 8>, 8, 256, -1, 0, 0)
-SPR_COL_VARIANT(1024, 7, RadixPlan<1024>, 8, 256, -1, 1, 1)
 SPR_COL_VARIANT(2048, 1, RadixPlan<2048>, 4, 256, -1, 0, 1)
 SPR_COL_VARIANT(2048, 2, Plan<2048, 16, 16, 8, 16>, 8, 256, -1, 0, 1)
-// (plan, columns, -, -, -, -, -, spare tile row every 2^k rows): tiles without
-// the bank conflicts of the padded layouts. Measured on MI355X the conflicts
-// cost little (the pass is bound by HBM and VALU): 768^2 4 columns 73.7 vs
-// 76.7 us, 1024^2 radix 16 8 columns 68.7 vs 69.6 us, 512^2 8 columns 56.6 vs
-// 57.4 us; at 256^2, 384^2 and 2048^2 the skewed tiles were slower.
+// (plan, columns, -, -, -, -, -, spare tile row every 2^k rows, waves per SIMD):
+// tiles without the bank conflicts of the padded layouts. Their address
+// arithmetic takes registers, which k_col_step lacks: with 80 (512^2, 8 columns)
+// it spills and the iteration takes 0.080 ms against 0.077 in the padded tile;
+// the plain projection pass is ahead in them (52 against 60 us).
 SPR_COL_VARIANT(512, 6, RadixPlan<512>, 8, 256, -1, 0, 0, 3, 3)
+SPR_COL_VARIANT(512, 7, RadixPlan<512>, 4, 256, -1, 0, 0, 3, 2, 5)
+SPR_COL_VARIANT(768, 1, RadixPlan<768>, 4, 256, -1, 1, 0, 3, 2, 3)
 SPR_COL_VARIANT(768, 6, RadixPlan<768>, 4, 256, -1, 0, 0, 3, 2)
-// (plan, columns, -, -, padding, -, -, -, column groups, waves per SIMD): strips
-// of 16 columns (whole 128-byte row segments) transformed as groups of 8 or 4
-// columns through one tile, so that one group's transforms overlap the next
-// group's loads and the previous group's stores
-SPR_COL_VARIANT(512, 7, RadixPlan<512>, 8, 256, -1, 1, 0, 3, 0, 2, 0)
-SPR_COL_VARIANT(768, 7, RadixPlan<768>, 8, 256, -1, 1, 0, 3, 0, 2, 4)
+SPR_COL_VARIANT(1024, 7, Plan<1024, 16, 16, 8, 8>, 4, 256, -1, 0, 0, 3, 4, 3)
 // row variants: plan, -, threads per workgroup, prefetch mode
 SPR_ROW_VARIANT(256, 1, RadixPlan<256>, 0, 512)
 SPR_ROW_VARIANT(384, 1, RadixPlan<384>, 0, 512)
@@ -194,21 +189,38 @@ SPR_ROW_VARIANT(512, 2, RadixPlan<512>, 0, 256, -1, 1, 0, 4)
 SPR_ROW_VARIANT(768, 3, RadixPlan<768>, 0, 256, -1, 1, 0, 5)
 SPR_ROW_VARIANT(1024, 5, RadixPlan<1024>, 0, 256, -1, 1, 0, 4)
 SPR_ROW_VARIANT(2048, 3, RadixPlan<2048>, 0, 256, -1, 1, 0, 4)
-// (plan, -, threads, prefetch, -, -, padding period, -, -, -, recomputed state):
-// the row update passes recompute rho_n from its row transform instead of
-// reading and writing it (one more row transform for 8 fewer bytes per pixel);
-// the column pass then writes its projection to a second field buffer
-SPR_ROW_VARIANT(256, 3, RadixPlan<256>, 0, 256, -1, 1, 0, 4, 0, 1, 0, 1)
-SPR_ROW_VARIANT(384, 3, RadixPlan<384>, 0, 256, -1, 1, 0, 5, 0, 1, 0, 1)
-SPR_ROW_VARIANT(512, 3, RadixPlan<512>, 0, 256, -1, 1, 0, 3, 0, 1, 0, 1)
-SPR_ROW_VARIANT(512, 4, RadixPlan<512>, 0, 256, -1, 1, 0, 4, 0, 1, 0, 1)
-SPR_ROW_VARIANT(768, 4, RadixPlan<768>, 0, 256, -1, 1, 0, 5, 0, 1, 0, 1)
-SPR_ROW_VARIANT(1024, 6, RadixPlan<1024>, 0, 256, -1, 1, 0, 4, 0, 1, 0, 1)
-SPR_ROW_VARIANT(1024, 7, Plan<1024, 16, 16, 8, 8>, 0, 256, -1, 1, 0, 3, 0, 1, 0, 1)
-SPR_ROW_VARIANT(2048, 4, RadixPlan<2048>, 0, 256, -1, 1, 0, 4, 0, 1, 0, 1)
-SPR_ROW_VARIANT(2048, 5, Plan<2048, 16, 16, 8, 16>, 0, 256, -1, 1, 0, 4, 0, 1, 0, 1)
+// (plan, -, threads, prefetch, -, -, padding period, -, -, recomputed state): the
+// row update passes recompute rho_n from its row transform instead of reading
+// and writing it, and run on the rows that meet the support (k_row_listed); the
+// column passes write their projection to a second field buffer (k_col_step)
+SPR_ROW_VARIANT(256, 3, RadixPlan<256>, 0, 256, -1, 1, 0, 4, 0, 0, 1)
+SPR_ROW_VARIANT(384, 3, RadixPlan<384>, 0, 256, -1, 1, 0, 5, 0, 0, 1)
+SPR_ROW_VARIANT(512, 3, RadixPlan<512>, 0, 256, -1, 1, 0, 3, 0, 0, 1)
+SPR_ROW_VARIANT(512, 4, RadixPlan<512>, 0, 256, -1, 1, 0, 4, 0, 0, 1)
+SPR_ROW_VARIANT(768, 4, RadixPlan<768>, 0, 256, -1, 1, 0, 5, 0, 0, 1)
+SPR_ROW_VARIANT(1024, 6, RadixPlan<1024>, 0, 256, -1, 1, 0, 4, 0, 0, 1)
+SPR_ROW_VARIANT(1024, 7, Plan<1024, 16, 16, 8, 8>, 0, 256, -1, 1, 0, 3, 0, 0, 1)
+SPR_ROW_VARIANT(2048, 4, RadixPlan<2048>, 0, 256, -1, 1, 0, 4, 0, 0, 1)
+SPR_ROW_VARIANT(2048, 5, Plan<2048, 16, 16, 8, 16>, 0, 256, -1, 1, 0, 4, 0, 0, 1)
 #undef SPR_COL_VARIANT
 #undef SPR_ROW_VARIANT
+
+// The column variant that k_col_step takes in place of CV while CV's strips leave
+// CUs without a workgroup: the same plan in tiles half as wide. At 512^2 x 1
+// (64 or 128 workgroups on 256 CUs) an iteration takes 11.1 instead of 12.2 us,
+// at 1024^2 x 1 17.8 instead of 19.0, at 384^2 x 1 13.7 instead of 14.2; from 256
+// workgroups on the wide tiles are even or ahead (512^2 x 4: 13.6 against 14.3).
+template <int N, int CV> constexpr int narrow_variant() {
+    if constexpr (N == 384 && CV == 1) return 3;
+    else if constexpr (N == 512 && CV == 1) return 7;
+    else if constexpr (N == 1024 && CV == 6) return 7;
+    else return CV;
+}
+
+// The column variant of the plain projection (k_col) in place of CV: the same plan
+// in the layout that pass runs best in, where it is not the step pass's. 512^2 x
+// 64: 52 us in the skewed tile, 60 in the padded one.
+template <int N, int CV> constexpr int plain_variant() { return N == 512 && CV == 1 ? 6 : CV; }
 
 constexpr int MAX_VARIANTS = 8;
 template <int N> constexpr int col_variants() {
@@ -395,6 +407,10 @@ struct RowArgs {
     PhaseCut pc;
     const float2* proj;  // column-projected fields, read by variants that recompute rho_n
     float inv_n;         // 1/N
+    // Rows that meet the support (variants that recompute rho_n): per field
+    // their number and, ascending, their indices.
+    const int* rowcnt;       // [fields]
+    const uint16_t* rowlist; // [fields][N]
 };
 
 // Support bit of pixel i of a field: bit i&31 of word i>>5 (N*N and the
@@ -403,11 +419,40 @@ __device__ __forceinline__ uint8_t support_bit(const uint32_t* __restrict__ bits
     return (uint8_t)((bits[i >> 5] >> (i & 31)) & 1u);
 }
 
-// supp (bytes) -> bits: word w holds pixels [32w, 32w+32), bit k = (supp[32w+k] != 0).
-// Each thread reads its 32 bytes as two 16-byte loads (supp 16-byte aligned).
-__global__ void k_pack_support(const uint8_t* __restrict__ supp, uint32_t* __restrict__ bits, size_t nwords) {
-    const size_t step = (size_t)gridDim.x * blockDim.x;
-    for (size_t w = (size_t)blockIdx.x * blockDim.x + threadIdx.x; w < nwords; w += step) {
+// The supports of a block in the forms its passes read, per field:
+//   bits     [N*N/32]  word w holds pixels [32w, 32w+32), bit k = (supp[32w+k] != 0)
+//   rowcnt             number of rows that meet the support
+//   rowlist  [N]       those rows, ascending
+//   colmask  [N/V]     bit q of entry t: row t + q*N/V meets the support (V values per
+//                      thread of the column pass, thread t of a column)
+// A field whose support is empty lists every row: its rows then run the general
+// update, which keeps the signs of zero that the projection of a vanishing
+// spectrum depends on.
+struct SupportPlan {
+    const uint8_t* supp;   // 16-byte aligned
+    uint32_t* bits;
+    int* rowcnt;
+    uint16_t* rowlist;
+    uint32_t* colmask;
+    uint32_t* rowflags;    // [N/32] one bit per row, from k_pack_support to k_row_plan
+    int n;
+    int lines;             // entries of colmask per field: N/V
+};
+
+// N/32 workgroups per field, 32 rows each: a thread packs 32 bytes at a time, as
+// two 16-byte loads. (One workgroup per field doing both kernels' work took 40 us
+// at 1024^2 x 32 and 14 us at 512^2 x 64; workgroups handing their flags to the
+// last one of the field 45 and 32 us, in agent-scope fences.)
+__global__ __launch_bounds__(256) void k_pack_support(SupportPlan a) {
+    __shared__ uint32_t hit;
+    const int tid = threadIdx.x, n = a.n, wpr = n / 32;
+    const size_t blk = blockIdx.x;   // field * wpr + 32-row group
+    const uint8_t* __restrict__ supp = a.supp + blk * 32 * n;
+    uint32_t* __restrict__ bits = a.bits + blk * n;
+    if (tid == 0) hit = 0;
+    __syncthreads();
+    uint32_t rows = 0;
+    for (int w = tid; w < n; w += 256) {
         const uint4 lo = *reinterpret_cast<const uint4*>(supp + 32 * w);
         const uint4 hi = *reinterpret_cast<const uint4*>(supp + 32 * w + 16);
         const unsigned x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
@@ -417,6 +462,43 @@ __global__ void k_pack_support(const uint8_t* __restrict__ supp, uint32_t* __res
 #pragma unroll
             for (int j = 0; j < 4; ++j) m |= (uint32_t)(((x[k] >> (8 * j)) & 0xffu) != 0u) << (4 * k + j);
         bits[w] = m;
+        if (m) rows |= 1u << (w / wpr);
+    }
+    if (rows) atomicOr(&hit, rows);
+    __syncthreads();
+    if (tid == 0) a.rowflags[blk] = hit;
+}
+
+// Row list and column masks of one field per workgroup.
+__global__ __launch_bounds__(256) void k_row_plan(SupportPlan a) {
+    __shared__ uint32_t fw[64];   // one bit per row (N <= 2048)
+    __shared__ int fbase[64];     // rows listed before each word
+    const int tid = threadIdx.x, n = a.n, wpr = n / 32;
+    const size_t p = blockIdx.x;
+    if (tid < 64) {   // running sum of the flag words in one wavefront
+        uint32_t f = tid < wpr ? a.rowflags[p * wpr + tid] : 0u;
+        if (__ballot(f != 0u) == 0) f = tid < wpr ? 0xffffffffu : 0u;
+        const int cnt = __popc(f);
+        int sum = cnt;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int u = __shfl_up(sum, o, 64);
+            if (tid >= o) sum += u;
+        }
+        fw[tid] = f;
+        fbase[tid] = sum - cnt;
+        if (tid == 63) a.rowcnt[p] = sum;
+    }
+    __syncthreads();
+    for (int y = tid; y < n; y += 256) {
+        const uint32_t f = fw[y >> 5];
+        if ((f >> (y & 31)) & 1u)
+            a.rowlist[p * n + fbase[y >> 5] + __popc(f & ((1u << (y & 31)) - 1u))] = (uint16_t)y;
+    }
+    for (int t = tid; t < a.lines; t += 256) {
+        uint32_t m = 0;
+        for (int y = t, q = 0; y < n; y += a.lines, ++q) m |= ((fw[y >> 5] >> (y & 31)) & 1u) << q;
+        a.colmask[p * a.lines + t] = m;
     }
 }
 
@@ -435,9 +517,7 @@ __global__ __launch_bounds__((RowVariant<N, RV>::G::ROW_THREADS)) void k_row(Row
     constexpr int V = G::V, T = G::T;
     constexpr int PREFETCH = G::ROW_PREFETCH >= 0 ? G::ROW_PREFETCH : SPR_ROW_PREFETCH;
     constexpr bool WV = T <= 64;   // every row inside one wavefront: no workgroup barriers
-    constexpr bool RS = G::ROW_RECOMPUTE;
-    static_assert(!RS || PREFETCH >= 1, "the recomputed state is transformed from its prefetched row");
-    __shared__ float2 tw[TwTableP<PL>::SIZE];
+        __shared__ float2 tw[TwTableP<PL>::SIZE];
     __shared__ float2 lds[G::RW * G::RS];
     const int tid = threadIdx.x;
     const int t = tid % T;
@@ -461,7 +541,7 @@ __global__ __launch_bounds__((RowVariant<N, RV>::G::ROW_THREADS)) void k_row(Row
 #pragma unroll
         for (int q = 0; q < V; ++q) dst[off + q * T] = v[q];
     } else if constexpr (MODE == ROW_FINAL || MODE == ROW_INV_INPLACE) {
-        const float2* src = (MODE == ROW_FINAL) ? (RS ? a.proj + blk : work) : rho;
+        const float2* src = (MODE == ROW_FINAL) ? work : rho;
 #pragma unroll
         for (int r = 0; r < V; ++r) v[r] = src[off + r * T];
         fft_line_p<PL, -1, WV>(v, acc, tw, t);
@@ -469,49 +549,14 @@ __global__ __launch_bounds__((RowVariant<N, RV>::G::ROW_THREADS)) void k_row(Row
         for (int q = 0; q < V; ++q) rho[off + q * T] = make_float2(v[q].x * a.inv_nn, v[q].y * a.inv_nn);
     } else {
         // The state and the support may be loaded with the field, before the
-        // transform, so that their latency hides behind it. With RS the field
-        // comes from proj and the state is recomputed from its row transform
-        // (work): rho_n = rowIFFT(rowFFT(rho_n)) / N, within float rounding.
+        // transform, so that their latency hides behind it.
         float2 bn[V];
         uint8_t sn[V];
-        const float2* __restrict__ fin = RS ? a.proj + blk : work;
 #pragma unroll
         for (int r = 0; r < V; ++r) {
-            v[r] = ld_stream(fin + off + r * T);
+            v[r] = ld_stream(work + off + r * T);
             if constexpr (PREFETCH >= 2) sn[r] = support_bit(sbits, off + r * T);
-            if constexpr (MODE != ROW_ER && PREFETCH >= 1) bn[r] = ld_stream((RS ? work : rho) + off + r * T);
-        }
-        if constexpr (RS && MODE == ROW_RAAR) {
-            // RAAR needs rho' and rho_n only through q = 2 rho' - rho_n: its
-            // rejected branch beta rho_n + (1 - 2 beta) rho' is rho' - beta q. The
-            // transforms are linear, so q is one inverse transform of
-            // 2 proj / N^2 - work / N, and the new row transform is
-            // rowFFT(rho') - beta rowFFT(c) = proj / N - beta rowFFT(c), with c = q
-            // on the rejected pixels and 0 elsewhere: two row transforms, as with
-            // the state stored.
-            const float two_nn = 2.f * a.inv_nn;
-#pragma unroll
-            for (int r = 0; r < V; ++r) {
-                const float2 pr = v[r], wr = bn[r];
-                v[r] = make_float2(two_nn * pr.x - a.inv_n * wr.x, two_nn * pr.y - a.inv_n * wr.y);
-                bn[r] = make_float2(a.inv_n * pr.x, a.inv_n * pr.y);
-            }
-            fft_line_p<PL, -1, WV>(v, acc, tw, t);   // q
-#pragma unroll
-            for (int q = 0; q < V; ++q) {
-                const uint8_t s = PREFETCH >= 2 ? sn[q] : support_bit(sbits, off + q * T);
-                if (s != 0 && !phase_fails(v[q].x, v[q].y, a.pc)) v[q] = make_float2(0.f, 0.f);
-            }
-            fft_line_p<PL, +1, WV>(v, acc, tw, t);   // rowFFT(c)
-#pragma unroll
-            for (int q = 0; q < V; ++q)
-                st_stream(work + off + q * T, make_float2(bn[q].x - a.beta * v[q].x, bn[q].y - a.beta * v[q].y));
-            return;
-        }
-        if constexpr (RS && MODE != ROW_ER) {
-            fft_line_p<PL, -1, WV>(bn, acc, tw, t);
-#pragma unroll
-            for (int r = 0; r < V; ++r) bn[r] = make_float2(bn[r].x * a.inv_n, bn[r].y * a.inv_n);
+            if constexpr (MODE != ROW_ER && PREFETCH >= 1) bn[r] = ld_stream(rho + off + r * T);
         }
         fft_line_p<PL, -1, WV>(v, acc, tw, t);
 #pragma unroll
@@ -537,10 +582,103 @@ __global__ __launch_bounds__((RowVariant<N, RV>::G::ROW_THREADS)) void k_row(Row
                     o = make_float2(a.beta * b.x + c * d.x, a.beta * b.y + c * d.y);
                 }
             }
-            if constexpr (MODE != ROW_ER && !RS) st_stream(rho + i, o);
+            if constexpr (MODE != ROW_ER) st_stream(rho + i, o);
             v[q] = o;
         }
         fft_line_p<PL, +1, WV>(v, acc, tw, t);
+#pragma unroll
+        for (int q = 0; q < V; ++q) st_stream(work + off + q * T, v[q]);
+    }
+}
+
+// Row update of an iteration that recomputes rho_n: the rows that meet the
+// support, RW at a time (the column pass, k_col_step, has updated the others).
+// Workgroup b takes field b % fields and group b / fields of its list; those past
+// the lists' ends come last and leave at once (workgroups that step through the
+// lists instead, twinned down to 4096, took the same time: 20 us at 512^2 x 64
+// with 22 % of the rows listed, against 60 us for the pass over every row).
+template <int N, int MODE, int RV>
+__global__ __launch_bounds__((RowVariant<N, RV>::G::ROW_THREADS)) void k_row_listed(RowArgs a, int fields) {
+    using G = typename RowVariant<N, RV>::G;
+    using PL = typename G::PL;
+    constexpr int V = G::V, T = G::T, RW = G::RW;
+    constexpr bool WV = T <= 64;   // every row inside one wavefront: no workgroup barriers
+    __shared__ float2 tw[TwTableP<PL>::SIZE];
+    __shared__ float2 lds[RW * G::RS];
+    const int tid = threadIdx.x;
+    const int t = tid % T;
+    const int rl = tid / T;
+    const int field = blockIdx.x % fields;
+    const int listed = a.rowcnt[field];
+    const int first = blockIdx.x / fields * RW;
+    if (first >= listed) return;
+    tw_fill_p<PL>(tw, a.tw, tid, G::ROW_THREADS);
+    // Block-uniform bases with 32-bit per-thread offsets (SGPR base addressing).
+    const size_t blk = (size_t)field * N * N;
+    float2* __restrict__ work = a.work + blk;
+    const uint32_t* __restrict__ sbits = a.sbits + blk / 32;
+    const uint16_t* __restrict__ list = a.rowlist + (size_t)field * N;
+    const RowAccT<G::ROW_PAD_SHIFT> acc{lds + rl * G::RS};
+    __syncthreads();
+    // Past the list's end a line repeats the last row and stores nothing.
+    const bool live = first + rl < listed;
+    const int off = list[live ? first + rl : listed - 1] * N + t;
+    float2 v[V];
+    // rho' = rowIFFT(proj)/N^2 and rho_n = rowIFFT(work)/N, the state recomputed
+    // from its row transform (within float rounding); ER needs rho' only, which
+    // its column pass leaves in work.
+    float2 bn[V];
+    uint8_t sn[V];
+    const float2* __restrict__ fin = MODE == ROW_ER ? work : a.proj + blk;
+#pragma unroll
+    for (int r = 0; r < V; ++r) {
+        v[r] = ld_stream(fin + off + r * T);
+        sn[r] = support_bit(sbits, off + r * T);
+        if constexpr (MODE != ROW_ER) bn[r] = ld_stream(work + off + r * T);
+    }
+    if constexpr (MODE == ROW_RAAR) {
+        // RAAR needs rho' and rho_n only through q = 2 rho' - rho_n: its
+        // rejected branch beta rho_n + (1 - 2 beta) rho' is rho' - beta q. The
+        // transforms are linear, so q is one inverse transform of
+        // 2 proj / N^2 - work / N, and the new row transform is
+        // rowFFT(rho') - beta rowFFT(c) = proj / N - beta rowFFT(c), with c = q
+        // on the rejected pixels and 0 elsewhere: two row transforms, as with
+        // the state stored.
+        const float two_nn = 2.f * a.inv_nn;
+#pragma unroll
+        for (int r = 0; r < V; ++r) {
+            const float2 pr = v[r], wr = bn[r];
+            v[r] = make_float2(two_nn * pr.x - a.inv_n * wr.x, two_nn * pr.y - a.inv_n * wr.y);
+            bn[r] = make_float2(a.inv_n * pr.x, a.inv_n * pr.y);
+        }
+        fft_line_p<PL, -1, WV>(v, acc, tw, t);   // q
+#pragma unroll
+        for (int q = 0; q < V; ++q)
+            if (sn[q] != 0 && !phase_fails(v[q].x, v[q].y, a.pc)) v[q] = make_float2(0.f, 0.f);
+        fft_line_p<PL, +1, WV>(v, acc, tw, t);   // rowFFT(c)
+#pragma unroll
+        for (int q = 0; q < V; ++q)
+            v[q] = make_float2(bn[q].x - a.beta * v[q].x, bn[q].y - a.beta * v[q].y);
+    } else {
+        if constexpr (MODE == ROW_HIO) {
+            fft_line_p<PL, -1, WV>(bn, acc, tw, t);
+#pragma unroll
+            for (int r = 0; r < V; ++r) bn[r] = make_float2(bn[r].x * a.inv_n, bn[r].y * a.inv_n);
+        }
+        fft_line_p<PL, -1, WV>(v, acc, tw, t);
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+            const float2 d = make_float2(v[q].x * a.inv_nn, v[q].y * a.inv_nn);  // rho'
+            const float ts = (sn[q] != 0 && !phase_fails(d.x, d.y, a.pc)) ? 1.f : 0.f;
+            if constexpr (MODE == ROW_ER)
+                v[q] = make_float2(d.x * ts, d.y * ts);
+            else
+                v[q] = make_float2((bn[q].x - a.beta * d.x) * (1.f - ts) + d.x * ts,
+                                   (bn[q].y - a.beta * d.y) * (1.f - ts) + d.y * ts);
+        }
+        fft_line_p<PL, +1, WV>(v, acc, tw, t);
+    }
+    if (live) {
 #pragma unroll
         for (int q = 0; q < V; ++q) st_stream(work + off + q * T, v[q]);
     }
@@ -609,25 +747,17 @@ __attribute__((amdgpu_waves_per_eu((ColVariant<N, CV>::G::COL_WAVES_PER_EU)))) v
     const float2* tw = twl;
     if constexpr (G::TW_GLOBAL) tw = a.twtab;
     else tw_fill_p<PL>(twl, a.tw, tid, G::COL_THREADS);
-    constexpr int CG = G::COL_GROUPS;
-    constexpr int TILES = N / G::COL_STRIP;
-    const int strip = col_strip<N, G::COL_STRIP>(blockIdx.x);
+    constexpr int TILES = N / C;
+    const int strip = col_strip<N, C>(blockIdx.x);
     const int p = strip / TILES;
-    const int x0 = (strip % TILES) * G::COL_STRIP;
+    const int x0 = (strip % TILES) * C;
     // Block-uniform bases with 32-bit per-thread offsets (SGPR base addressing).
     float2* __restrict__ f = a.f + (size_t)p * N * N + x0;
     float2* __restrict__ fo = a.out + (size_t)p * N * N + x0;
     const int off = t * N + c;
-    // Group g of the strip is columns [g*C, (g+1)*C). The loads are issued
-    // group after group, so that the wait for group 0's values leaves the later
-    // groups' loads in flight during group 0's transforms (the other half of
-    // each line comes from the L2).
-    float2 vg[CG][V];
+    float2 v[V];
 #pragma unroll
-    for (int g = 0; g < CG; ++g)
-#pragma unroll
-        for (int r = 0; r < V; ++r) vg[g][r] = ld_stream(f + off + g * C + r * T * N);
-    float2(&v)[V] = vg[0];
+    for (int r = 0; r < V; ++r) v[r] = ld_stream(f + off + r * T * N);
     if constexpr (WV) {
         constexpr int CST = G::CST;
         const int cc = tid / T;   // column owned by this thread's wavefront
@@ -655,39 +785,147 @@ __attribute__((amdgpu_waves_per_eu((ColVariant<N, CV>::G::COL_WAVES_PER_EU)))) v
         const float* __restrict__ amp = a.amp + amp_offset<N>(a.amp_of, p) + x0;
         using Acc = std::conditional_t<(G::COL_SKEW > 0), ColAccSkew<C, (G::COL_SKEW > 0 ? G::COL_SKEW : 1)>, ColAcc<CS>>;
         const Acc acc{lds + c};
-        // The amplitude of group 0 is loaded with the field; that of a later
-        // group when its turn starts, so that its latency hides behind the
-        // group's forward transform while only one group's values are live.
         float am[V];
         if constexpr (MODE == COL_PROJ && SPR_COL_AMP_PREFETCH) {
 #pragma unroll
             for (int q = 0; q < V; ++q) am[q] = amp[off + q * T * N];
         }
         __syncthreads();
+        if constexpr (MODE == COL_PROJ || MODE == COL_FWD) fft_line_p<PL, +1>(v, acc, tw, t);
+        if constexpr (MODE == COL_PROJ) {
 #pragma unroll
-        for (int g = 0; g < CG; ++g) {
-            if constexpr (MODE == COL_PROJ && SPR_COL_AMP_PREFETCH) {
-                if (g > 0) {
-#pragma unroll
-                    for (int q = 0; q < V; ++q) am[q] = amp[off + g * C + q * T * N];
-                }
-            }
-            if constexpr (MODE == COL_PROJ || MODE == COL_FWD) fft_line_p<PL, +1>(vg[g], acc, tw, t);
-            if constexpr (MODE == COL_PROJ) {
-#pragma unroll
-                for (int q = 0; q < V; ++q)
-                    vg[g][q] = project_modulus(vg[g][q], SPR_COL_AMP_PREFETCH ? am[q] : amp[off + g * C + q * T * N]);
-            }
-            if constexpr (MODE == COL_PROJ || MODE == COL_INV) fft_line_p<PL, -1>(vg[g], acc, tw, t);
-            if constexpr (CG > 1) {
-#pragma unroll
-                for (int q = 0; q < V; ++q) st_stream(fo + off + g * C + q * T * N, vg[g][q]);
-            }
+            for (int q = 0; q < V; ++q)
+                v[q] = project_modulus(v[q], SPR_COL_AMP_PREFETCH ? am[q] : amp[off + q * T * N]);
         }
-        if constexpr (CG > 1) return;
+        if constexpr (MODE == COL_PROJ || MODE == COL_INV) fft_line_p<PL, -1>(v, acc, tw, t);
     }
 #pragma unroll
     for (int q = 0; q < V; ++q) st_stream(fo + off + q * T * N, v[q]);
+}
+
+// ---------------------------------------------------------------------------
+// Projection pass of an iteration that recomputes rho_n, by rows that meet the
+// support or not
+// ---------------------------------------------------------------------------
+enum StepMode {
+    STEP_LIN = 0,      // HIO, RAAR: proj <- projected rows that meet the support; f <- the update of the others
+    STEP_ER = 1,       // f <- projected rows that meet the support; the others are 0 in the next iteration
+    STEP_ER_LAST = 2,  // f <- every projected row (trailing projection; its input rows as STEP_ER's)
+};
+
+struct StepArgs {
+    float2* f;          // [fields][N][N] row transforms of rho_n
+    float2* proj;       // [fields][N][N] (STEP_LIN)
+    const float* amp;   // amplitudes [patterns][N][N]
+    const int* amp_of;  // field -> pattern (NULL: pattern 0)
+    const float2* twtab;      // the plan's twiddle table
+    const uint32_t* colmask;  // [fields][N/V] row masks of k_pack_support
+    float lin_w, lin_p;       // STEP_LIN: f <- lin_w f + lin_p projected outside the support
+    int all_rows;             // STEP_ER*: rho_n is any density (the first pass of a block)
+};
+
+// One field of N*N elements of E bytes as a raw buffer: addresses are a 32-bit
+// per-thread offset plus a scalar one, so the V rows of a thread cost no address
+// arithmetic on the vector ALUs, which bound the column passes; an offset with
+// the top bit set is out of range: it reads 0 and writes nothing.
+template <int N, int E> __device__ __forceinline__ __amdgpu_buffer_rsrc_t field_buffer(const void* base) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, N * N * E, 0x00027000);
+}
+using u32x2 = unsigned __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float2 buf_ld2(__amdgpu_buffer_rsrc_t b, int voff, int soff) {
+    const u32x2 x = __builtin_amdgcn_raw_buffer_load_b64(b, voff, soff, 0);
+    return make_float2(__uint_as_float(x.x), __uint_as_float(x.y));
+}
+__device__ __forceinline__ float buf_ld1(__amdgpu_buffer_rsrc_t b, int voff, int soff) {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b, voff, soff, 0));
+}
+__device__ __forceinline__ void buf_st2(__amdgpu_buffer_rsrc_t b, float2 v, int voff, int soff) {
+    u32x2 x;
+    x.x = __float_as_uint(v.x);
+    x.y = __float_as_uint(v.y);
+    __builtin_amdgcn_raw_buffer_store_b64(x, b, voff, soff, 0);
+}
+// voff, out of range where bit q of `off_rows` is set.
+__device__ __forceinline__ int row_offset(int voff, uint32_t off_rows, int q) {
+    return voff | (int)((off_rows << (31 - q)) & 0x80000000u);
+}
+
+// Columns [x0, x0 + C) of one field. Outside the support (s = 0) the update is
+// linear in rho_n and rho', so it can be made on their row transforms, f and
+// proj/N = rowFFT(rho'):
+//   HIO   rho_n - beta rho'              f <- f - (beta/N) proj
+//   RAAR  beta rho_n + (1-2 beta) rho'   f <- beta f + ((1-2 beta)/N) proj
+//   ER    0
+// A row without a support pixel is updated here, in place, from registers: 16
+// B/px for the pass, as for the plain projection, and the row pass (24 B/px and
+// two or three transforms) visits only the rows that meet the support, 10 - 45 %
+// of them for objects on an oversampled grid.
+template <int N, int MODE, int CV>
+__global__ __launch_bounds__((ColVariant<N, CV>::G::COL_THREADS))
+__attribute__((amdgpu_waves_per_eu((ColVariant<N, CV>::G::COL_WAVES_PER_EU)))) void k_col_step(StepArgs a) {
+    using G = typename ColVariant<N, CV>::G;
+    using PL = typename G::PL;
+    constexpr int V = G::V, T = G::T, C = G::C;
+    __shared__ float2 twl[G::TW_GLOBAL ? 1 : TwTableP<PL>::SIZE];
+    __shared__ float2 lds[G::COL_TILE];
+    const int tid = threadIdx.x;
+    const int c = tid % C;
+    const int t = tid / C;
+    constexpr int TILES = N / C;
+    const int strip = col_strip<N, C>(blockIdx.x);
+    const int p = strip / TILES;
+    const int x0 = (strip % TILES) * C;
+    const uint32_t off_rows = ~a.colmask[(size_t)p * T + t];
+    const float2* tw = twl;
+    if constexpr (G::TW_GLOBAL) {
+        tw = a.twtab;
+    } else {
+        for (int e = tid; e < TwTableP<PL>::SIZE; e += G::COL_THREADS) twl[e] = a.twtab[e];
+    }
+    const __amdgpu_buffer_rsrc_t bf = field_buffer<N, 8>(a.f + (size_t)p * N * N);
+    const __amdgpu_buffer_rsrc_t ba = field_buffer<N, 4>(a.amp + amp_offset<N>(a.amp_of, p));
+    const int off = t * N + x0 + c;
+    using Acc = std::conditional_t<(G::COL_SKEW > 0), ColAccSkew<C, (G::COL_SKEW > 0 ? G::COL_SKEW : 1)>, ColAcc<G::CS>>;
+    const Acc acc{lds + c};
+    float2 v[V], w[V];
+    const uint32_t skip = MODE == STEP_LIN || a.all_rows ? 0u : off_rows;
+#pragma unroll
+    for (int r = 0; r < V; ++r) v[r] = buf_ld2(bf, row_offset(8 * off, skip, r), 8 * r * T * N);
+    if constexpr (MODE == STEP_LIN) {
+#pragma unroll
+        for (int r = 0; r < V; ++r) w[r] = v[r];
+    }
+    // The amplitude, shared by all fields and resident in the L2: with f where it
+    // fits in the registers beside w, else after the transform.
+    constexpr bool AMP_EARLY = V <= 8;
+    float am[V];
+    auto load_amp = [&]() {
+#pragma unroll
+        for (int q = 0; q < V; ++q) am[q] = buf_ld1(ba, 4 * off, 4 * q * T * N);
+    };
+    if constexpr (AMP_EARLY) load_amp();
+    __syncthreads();   // twiddle table
+    fft_line_p<PL, +1>(v, acc, tw, t);
+    if constexpr (!AMP_EARLY) load_amp();
+#pragma unroll
+    for (int q = 0; q < V; ++q) v[q] = project_modulus(v[q], am[q]);
+    fft_line_p<PL, -1>(v, acc, tw, t);
+    if constexpr (MODE == STEP_LIN) {
+        const __amdgpu_buffer_rsrc_t bp = field_buffer<N, 8>(a.proj + (size_t)p * N * N);
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+            // a wavefront holds a few adjacent rows: mostly one side only
+            if ((off_rows >> q) & 1u)
+                buf_st2(bf, make_float2(a.lin_w * w[q].x + a.lin_p * v[q].x, a.lin_w * w[q].y + a.lin_p * v[q].y),
+                        8 * off, 8 * q * T * N);
+            else
+                buf_st2(bp, v[q], 8 * off, 8 * q * T * N);
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < V; ++q)
+            buf_st2(bf, v[q], row_offset(8 * off, MODE == STEP_ER ? off_rows : 0u, q), 8 * q * T * N);
+    }
 }
 
 }  // namespace spr

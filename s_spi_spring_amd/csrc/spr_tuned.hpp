@@ -9,11 +9,11 @@ struct TunedVariants {
     int n, col, row;
 };
 constexpr TunedVariants kTuned[] = {
-    {256, 1, 3},
+    {256, 2, 3},
     {384, 1, 3},
-    {512, 6, 3},
-    {768, 4, 4},
-    {1024, 4, 6},
+    {512, 1, 3},
+    {768, 2, 4},
+    {1024, 6, 6},
     {2048, 2, 5},
 };
 
