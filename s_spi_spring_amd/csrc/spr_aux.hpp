@@ -80,6 +80,13 @@ __device__ __forceinline__ unsigned long long block_max_u64(unsigned long long v
     return v;
 }
 
+// Column passes outside the iteration: tiles of 8 columns where the default is
+// wider, 16 up to 128^2 (whole 128-byte lines). A workgroup then has 4 - 8
+// wavefronts instead of 16, so that the correlation passes, which hold two fields'
+// values (94 registers), keep 3 - 4 workgroups on a CU instead of one.
+template <int N> constexpr int aux_columns() { return N <= 128 ? 16 : Geo<N>::C < 8 ? Geo<N>::C : 8; }
+template <int N> using AuxGeo = GeoT<N, RadixPlan<N>, aux_columns<N>()>;
+
 // ---------------------------------------------------------------------------
 // Spectral windows
 // ---------------------------------------------------------------------------
@@ -114,6 +121,15 @@ template <int N> __device__ __forceinline__ float corr_weight(int ix, int iy, co
     const float coeffmax = effmax > 0 ? expf(-effmax * effmax / w.sigmax2) : 1.f;
     coeff *= coeffmax;
     return coeff * coeff;
+}
+
+// The window of every frequency, once per operation: a pixel's weight costs two
+// exponentials, a square root and a double subtraction, and the correlation
+// passes need it twice for every field (at 512^2 x 64 they took 220 us for 24
+// B/px computing it; as a table of N^2 floats it stays in the L2).
+template <int N> __global__ __launch_bounds__(256) void k_corr_window(CorrWin w, float* out) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < N * N) out[i] = corr_weight<N>(i % N, i / N, w);
 }
 
 // ---------------------------------------------------------------------------
@@ -200,11 +216,11 @@ __global__ __launch_bounds__(Geo<N>::ROW_THREADS) void k_row_aux(AuxRowArgs a) {
             if (m > 0.f) ms[0] += (double)m;
             v[r] = d;
         }
-        block_sum<1, NT>(ms, red);
-        if (tid == 0) a.partial[blockIdx.x] = ms[0];
         fft_line<N, +1, (G::T <= 64)>(v, acc, tw, t);
 #pragma unroll
         for (int q = 0; q < V; ++q) a.work[base + t + q * T] = v[q];
+        block_sum<1, NT>(ms, red);
+        if (tid == 0) a.partial[blockIdx.x] = ms[0];
     } else if constexpr (MODE == AROW_ERR_REAL) {
 #pragma unroll
         for (int r = 0; r < V; ++r) v[r] = a.work[base + t + r * T];
@@ -285,13 +301,28 @@ struct AuxColArgs {
     unsigned* maxbits;
     const float2* ref;          // ACOL_CORR reference spectra (base of a batch)
     const int* ref_index;       // item -> reference spectrum (NULL: the item's own transformed field)
-    CorrWin win;
+    const float* win;           // ACOL_CORR: k_corr_window's table
     int unit_scale;             // ACOL_CORR: apply normalize_ft_shift to d first
 };
 
+// normalize_ft_shift with e = 1: z |z|/|z|.
+__device__ __forceinline__ float2 unit_scaled(float2 z) {
+    const float m = sqrtf(z.x * z.x + z.y * z.y);
+    const float s = m / m;
+    return make_float2(z.x * s, z.y * s);
+}
+// (re d, sg im d) r, weighted; 0 at masked pixels.
+__device__ __forceinline__ float2 corr_product(float2 d, float2 r, float sg, float w, bool masked) {
+    float cx = d.x * r.x - (sg * d.y) * r.y;
+    float cy = d.x * r.y + (sg * d.y) * r.x;
+    cx *= w;
+    cy *= w;
+    return masked ? make_float2(0.f, 0.f) : make_float2(cx, cy);
+}
+
 template <int N, int MODE>
-__global__ __launch_bounds__(Geo<N>::COL_THREADS) void k_col_aux(AuxColArgs a) {
-    using G = Geo<N>;
+__global__ __launch_bounds__(AuxGeo<N>::COL_THREADS) void k_col_aux(AuxColArgs a) {
+    using G = AuxGeo<N>;
     constexpr int V = G::V, T = G::T, C = G::C, NT = G::COL_THREADS;
     __shared__ float2 tw[TwTable<N>::SIZE];
     __shared__ float2 lds[N * G::CS];
@@ -301,7 +332,7 @@ __global__ __launch_bounds__(Geo<N>::COL_THREADS) void k_col_aux(AuxColArgs a) {
     const int t = tid / C;
     tw_fill<N>(tw, a.tw, tid, NT);
     constexpr int TILES = N / C;
-    const int strip = col_strip<N>(blockIdx.x);
+    const int strip = col_strip<N, C>(blockIdx.x);
     const int item = strip / TILES;
     const int x0 = (strip % TILES) * C;
     const size_t base = (size_t)item * N * N + x0 + c;
@@ -337,6 +368,9 @@ __global__ __launch_bounds__(Geo<N>::COL_THREADS) void k_col_aux(AuxColArgs a) {
             }
             v[q] = project_modulus(v[q], A);
         }
+        fft_line<N, -1>(v, acc, tw, t);
+#pragma unroll
+        for (int q = 0; q < V; ++q) a.f[base + (size_t)(t + q * T) * N] = v[q];
         block_sum<2, NT>(s, red);
         if (tid == 0) {
             a.partial[2 * strip] = s[0];
@@ -344,54 +378,33 @@ __global__ __launch_bounds__(Geo<N>::COL_THREADS) void k_col_aux(AuxColArgs a) {
         }
         fmax = block_max<NT>(fmax, reinterpret_cast<float*>(red));
         if (tid == 0) atomicMax(&a.maxbits[item], __float_as_uint(fmax));
-        fft_line<N, -1>(v, acc, tw, t);
-#pragma unroll
-        for (int q = 0; q < V; ++q) a.f[base + (size_t)(t + q * T) * N] = v[q];
     } else if constexpr (MODE == ACOL_FWD_UNIT) {
 #pragma unroll
         for (int q = 0; q < V; ++q) {
-            const float m = sqrtf(v[q].x * v[q].x + v[q].y * v[q].y);
-            const float s = m / m;
-            a.f[base + (size_t)(t + q * T) * N] = make_float2(v[q].x * s, v[q].y * s);
+            a.f[base + (size_t)(t + q * T) * N] = unit_scaled(v[q]);
         }
     } else if constexpr (MODE == ACOL_CORR) {
-        float2 d[V];
+        // Both products at once, so that d, r, the window and the mask are read once
+        // and only the second product waits in registers:
+        // sign -1: (conj d) r ; sign +1: d r ; both weighted and masked.
+        float2 v2[V];
+        const float2* __restrict__ ref = a.ref ? a.ref + (size_t)(a.ref_index ? a.ref_index[item] : 0) * N * N + x0 + c : nullptr;
 #pragma unroll
         for (int q = 0; q < V; ++q) {
-            d[q] = v[q];
-            if (a.unit_scale) {
-                const float m = sqrtf(d[q].x * d[q].x + d[q].y * d[q].y);
-                const float s = m / m;
-                d[q] = make_float2(d[q].x * s, d[q].y * s);
-            }
+            const int ky = t + q * T;
+            const float2 d = a.unit_scale ? unit_scaled(v[q]) : v[q];
+            const float2 r = ref ? ref[(size_t)ky * N] : d;   // symmetry: the spectrum with itself
+            const float w = a.win[(size_t)ky * N + x0 + c];
+            const bool masked = amp[(size_t)ky * N + x0 + c] < 0.f;
+            v[q] = corr_product(d, r, -1.f, w, masked);
+            v2[q] = corr_product(d, r, 1.f, w, masked);
         }
-        // sign -1: (conj d) * r ; sign +1: d * r ; both weighted and masked
-        // (one loop body: unrolling it would hold both products' operands at once)
-#pragma unroll 1
-        for (int sgn = 0; sgn < 2; ++sgn) {
-            const float sg = sgn == 0 ? -1.f : 1.f;
+        fft_line<N, -1>(v, acc, tw, t);
 #pragma unroll
-            for (int q = 0; q < V; ++q) {
-                const int ky = t + q * T;
-                float2 r;
-                if (a.ref_index) r = a.ref[(size_t)a.ref_index[item] * N * N + (size_t)ky * N + x0 + c];
-                else r = d[q];   // symmetry: correlate the spectrum with itself
-                float cx = d[q].x * r.x - (sg * d[q].y) * r.y;
-                float cy = d[q].x * r.y + (sg * d[q].y) * r.x;
-                const float w = corr_weight<N>(x0 + c, ky, a.win);
-                cx *= w;
-                cy *= w;
-                if (amp[(size_t)ky * N + x0 + c] < 0.f) {
-                    cx = 0.f;
-                    cy = 0.f;
-                }
-                v[q] = make_float2(cx, cy);
-            }
-            fft_line<N, -1>(v, acc, tw, t);
-            float2* dst = sgn == 0 ? a.f : a.f2;
+        for (int q = 0; q < V; ++q) a.f[base + (size_t)(t + q * T) * N] = v[q];
+        fft_line<N, -1>(v2, acc, tw, t);
 #pragma unroll
-            for (int q = 0; q < V; ++q) dst[base + (size_t)(t + q * T) * N] = v[q];
-        }
+        for (int q = 0; q < V; ++q) a.f2[base + (size_t)(t + q * T) * N] = v2[q];
     }
 }
 
@@ -539,14 +552,14 @@ __global__ __launch_bounds__(Geo<N>::ROW_THREADS) void k_fft_rows(FieldBatch b) 
 
 // Column transforms (all columns of each listed field), in place.
 template <int N, int SIGN>
-__global__ __launch_bounds__(Geo<N>::COL_THREADS) void k_fft_cols(FieldBatch b) {
-    using G = Geo<N>;
+__global__ __launch_bounds__(AuxGeo<N>::COL_THREADS) void k_fft_cols(FieldBatch b) {
+    using G = AuxGeo<N>;
     constexpr int V = G::V, T = G::T, C = G::C, NT = G::COL_THREADS, TILES = N / C;
     __shared__ float2 tw[TwTable<N>::SIZE];
     __shared__ float2 lds[N * G::CS];
     const int tid = threadIdx.x, c = tid % C, t = tid / C;
     tw_fill<N>(tw, b.tw, tid, NT);
-    const int strip = col_strip<N>(blockIdx.x);
+    const int strip = col_strip<N, C>(blockIdx.x);
     const int item = strip / TILES;
     const int x0 = (strip % TILES) * C;
     float2* __restrict__ f = b.base + field_of(b, item) * N * N + x0;
@@ -573,25 +586,19 @@ struct CorrSpecArgs {
     float2* out2;
     const float* amp;
     const float2* tw;
-    CorrWin win;
+    const float* win;       // k_corr_window's table
     int unit_scale;         // apply normalize_ft_shift (z *= |z|/|z|) to d and r first
 };
 
-__device__ __forceinline__ float2 unit_scaled(float2 z) {
-    const float m = sqrtf(z.x * z.x + z.y * z.y);
-    const float s = m / m;
-    return make_float2(z.x * s, z.y * s);
-}
-
 template <int N>
-__global__ __launch_bounds__(Geo<N>::COL_THREADS) void k_corr_spec_cols(CorrSpecArgs a) {
-    using G = Geo<N>;
+__global__ __launch_bounds__(AuxGeo<N>::COL_THREADS) void k_corr_spec_cols(CorrSpecArgs a) {
+    using G = AuxGeo<N>;
     constexpr int V = G::V, T = G::T, C = G::C, NT = G::COL_THREADS, TILES = N / C;
     __shared__ float2 tw[TwTable<N>::SIZE];
     __shared__ float2 lds[N * G::CS];
     const int tid = threadIdx.x, c = tid % C, t = tid / C;
     tw_fill<N>(tw, a.tw, tid, NT);
-    const int strip = col_strip<N>(blockIdx.x);
+    const int strip = col_strip<N, C>(blockIdx.x);
     const int item = strip / TILES;
     const int x0 = (strip % TILES) * C;
     const float2* __restrict__ d = a.spec + (size_t)a.d_index[item] * N * N + x0;
@@ -600,34 +607,27 @@ __global__ __launch_bounds__(Geo<N>::COL_THREADS) void k_corr_spec_cols(CorrSpec
     const int off = t * N + c;
     const ColAcc<G::CS> acc{lds + c};
     __syncthreads();
+    float2 v[V], v2[V];   // both products at once, as in ACOL_CORR
 #pragma unroll
-    for (int sgn = 0; sgn < 2; ++sgn) {
-        const float sg = sgn == 0 ? -1.f : 1.f;
-        float2 v[V];
-#pragma unroll
-        for (int q = 0; q < V; ++q) {
-            const int ky = t + q * T;
-            float2 dv = d[off + q * T * N], rv = r[off + q * T * N];
-            if (a.unit_scale) {
-                dv = unit_scaled(dv);
-                rv = unit_scaled(rv);
-            }
-            float cx = dv.x * rv.x - (sg * dv.y) * rv.y;
-            float cy = dv.x * rv.y + (sg * dv.y) * rv.x;
-            const float w = corr_weight<N>(x0 + c, ky, a.win);
-            cx *= w;
-            cy *= w;
-            if (amp[off + q * T * N] < 0.f) {
-                cx = 0.f;
-                cy = 0.f;
-            }
-            v[q] = make_float2(cx, cy);
+    for (int q = 0; q < V; ++q) {
+        float2 dv = d[off + q * T * N], rv = r[off + q * T * N];
+        if (a.unit_scale) {
+            dv = unit_scaled(dv);
+            rv = unit_scaled(rv);
         }
-        fft_line<N, -1>(v, acc, tw, t);
-        float2* __restrict__ o = (sgn == 0 ? a.out1 : a.out2) + (size_t)item * N * N + x0;
-#pragma unroll
-        for (int q = 0; q < V; ++q) o[off + q * T * N] = v[q];
+        const float w = a.win[x0 + off + q * T * N];
+        const bool masked = amp[off + q * T * N] < 0.f;
+        v[q] = corr_product(dv, rv, -1.f, w, masked);
+        v2[q] = corr_product(dv, rv, 1.f, w, masked);
     }
+    float2* __restrict__ o1 = a.out1 + (size_t)item * N * N + x0;
+    float2* __restrict__ o2 = a.out2 + (size_t)item * N * N + x0;
+    fft_line<N, -1>(v, acc, tw, t);
+#pragma unroll
+    for (int q = 0; q < V; ++q) o1[off + q * T * N] = v[q];
+    fft_line<N, -1>(v2, acc, tw, t);
+#pragma unroll
+    for (int q = 0; q < V; ++q) o2[off + q * T * N] = v2[q];
 }
 
 // ---------------------------------------------------------------------------

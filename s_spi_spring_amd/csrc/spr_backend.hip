@@ -62,6 +62,7 @@ struct spr_ctx {
     uint32_t* colmask = nullptr;  // [cap][n/V], V >= 8 values per thread of the column pass
     uint32_t* rowflags = nullptr; // [cap][n/32]
     float* amp = nullptr;         // amplitudes [npat][n][n]
+    float* corrwin = nullptr;     // [n][n] correlation window of the current operation
     float* amp_t = nullptr;       // amp transposed (read along columns by the column pass)
     int npat = 1;                 // patterns sharing this handle (one amplitude each)
     int colvar = 0, rowvar = 0;   // variants of the column and row iteration passes
@@ -446,7 +447,7 @@ template <int N> int launch_row_aux(spr_ctx* c, int mode, const AuxRowArgs& a, i
 }
 
 template <int N> int launch_col_aux(spr_ctx* c, int mode, const AuxColArgs& a, int items) {
-    const dim3 grid((unsigned)((size_t)items * (N / Geo<N>::C))), block(Geo<N>::COL_THREADS);
+    const dim3 grid((unsigned)((size_t)items * (N / AuxGeo<N>::C))), block(AuxGeo<N>::COL_THREADS);
     switch (mode) {
         case ACOL_BLUR: hipLaunchKernelGGL((k_col_aux<N, ACOL_BLUR>), grid, block, 0, c->stream, a); break;
         case ACOL_ERR: hipLaunchKernelGGL((k_col_aux<N, ACOL_ERR>), grid, block, 0, c->stream, a); break;
@@ -476,6 +477,14 @@ int cols_per_wg(int n) {
 #define SPR_C_CASE(N_) if (n == N_) return Geo<N_>::C;
     SPR_SIZES(SPR_C_CASE)
 #undef SPR_C_CASE
+    return 1;
+}
+
+// Columns per workgroup of the auxiliary column passes.
+int aux_cols_per_wg(int n) {
+#define SPR_AC_CASE(N_) if (n == N_) return AuxGeo<N_>::C;
+    SPR_SIZES(SPR_AC_CASE)
+#undef SPR_AC_CASE
     return 1;
 }
 
@@ -625,10 +634,20 @@ int queue_error(spr_ctx* c, float reality) {
     AuxColArgs ca = aux_col_args(c);
     SPR_TRY2(fill_u32(c, c->maxbits, 0u, c->P));
     SPR_TRY2(col_aux(c, ACOL_ERR, ca, c->P));
-    SPR_TRY2(reduce(c, n / cols_per_wg(n), 2, 1, c->P));
+    SPR_TRY2(reduce(c, n / aux_cols_per_wg(n), 2, 1, c->P));
     SPR_TRY2(row_aux(c, AROW_ERR_REAL, a, c->P));
     SPR_TRY2(reduce(c, n / rows_per_wg(n), 2, 3, c->P));
     return SPR_OK;
+}
+
+template <int N> int launch_corr_window(spr_ctx* c, const CorrWin& w) {
+    hipLaunchKernelGGL((k_corr_window<N>), dim3(N * N / 256), dim3(256), 0, c->stream, w, c->corrwin);
+    SPR_HIP(c, hipGetLastError());
+    return SPR_OK;
+}
+// The window table of an operation's correlations, before the first of them.
+int corr_window(spr_ctx* c, float minr, float maxr) {
+    SPR_DISPATCH_N(c, launch_corr_window, c, make_corr_win(c->n, minr, maxr));
 }
 
 // Symmetry correlation maxima into keys (key1: conj(a) a, key2: a a).
@@ -637,7 +656,8 @@ int queue_symmetry(spr_ctx* c, float symmin, float symmax) {
     a.src = c->rho;
     SPR_TRY2(row_aux(c, AROW_ABS_FWD_RHO, a, c->P));
     AuxColArgs ca = aux_col_args(c);
-    ca.win = make_corr_win(c->n, symmin, symmax);
+    SPR_TRY2(corr_window(c, symmin, symmax));
+    ca.win = c->corrwin;
     ca.unit_scale = 1;
     ca.ref = nullptr;
     ca.ref_index = nullptr;
@@ -853,7 +873,7 @@ template <int N> int launch_fft_rows(spr_ctx* c, int sign, FieldBatch b, int ite
     return SPR_OK;
 }
 template <int N> int launch_fft_cols(spr_ctx* c, int sign, FieldBatch b, int items) {
-    const dim3 grid((unsigned)((size_t)items * (N / Geo<N>::C))), block(Geo<N>::COL_THREADS);
+    const dim3 grid((unsigned)((size_t)items * (N / AuxGeo<N>::C))), block(AuxGeo<N>::COL_THREADS);
     if (sign > 0) hipLaunchKernelGGL((k_fft_cols<N, +1>), grid, block, 0, c->stream, b);
     else hipLaunchKernelGGL((k_fft_cols<N, -1>), grid, block, 0, c->stream, b);
     SPR_HIP(c, hipGetLastError());
@@ -862,8 +882,8 @@ template <int N> int launch_fft_cols(spr_ctx* c, int sign, FieldBatch b, int ite
 template <int N> int launch_corr_spec(spr_ctx* c, CorrSpecArgs a, int items) {
     a.amp = c->amp;
     a.tw = c->tw;
-    hipLaunchKernelGGL((k_corr_spec_cols<N>), dim3((unsigned)((size_t)items * (N / Geo<N>::C))),
-                       dim3(Geo<N>::COL_THREADS), 0, c->stream, a);
+    hipLaunchKernelGGL((k_corr_spec_cols<N>), dim3((unsigned)((size_t)items * (N / AuxGeo<N>::C))),
+                       dim3(AuxGeo<N>::COL_THREADS), 0, c->stream, a);
     SPR_HIP(c, hipGetLastError());
     return SPR_OK;
 }
@@ -908,20 +928,9 @@ int modulus_spectra(spr_ctx* c, const float2* src, const int* src_index, float2*
     return fft_cols(c, +1, b, items);
 }
 
-// Correlate spectra d_index[i] against r_index[i], pick the shifts and write
-// them to shiftp (first index of the strict maximum, direct vs twin).
-int correlate_and_pick(spr_ctx* c, const float2* spec, const int* d_index, const int* r_index, float minr,
-                       float maxr, int unit_scale, const float* pdirect, const float* pflip, ShiftParam* shiftp,
-                       int items) {
-    CorrSpecArgs ca{};
-    ca.spec = spec;
-    ca.d_index = d_index;
-    ca.r_index = r_index;
-    ca.out1 = c->work;
-    ca.out2 = c->work2;
-    ca.win = make_corr_win(c->n, minr, maxr);
-    ca.unit_scale = unit_scale;
-    SPR_TRY2(corr_spec(c, ca, items));
+// The shifts of `items` correlations in work (direct) and work2 (twin): their row
+// transforms, the first index of the strict maximum, direct vs twin.
+int pick_shifts(spr_ctx* c, const float* pdirect, const float* pflip, ShiftParam* shiftp, int items) {
     SPR_TRY2(fill_u64(c, c->keys, 0ull, 2 * (size_t)c->cap));
     AuxRowArgs a = aux_row_args(c);
     SPR_TRY2(row_aux(c, AROW_CORR, a, items));
@@ -930,6 +939,24 @@ int correlate_and_pick(spr_ctx* c, const float2* spec, const int* d_index, const
                        pflip, c->n, shiftp, items);
     SPR_HIP(c, hipGetLastError());
     return SPR_OK;
+}
+
+// Correlate spectra d_index[i] against r_index[i] in the window of corr_window,
+// pick the shifts and write them to shiftp (first index of the strict maximum,
+// direct vs twin).
+int correlate_and_pick(spr_ctx* c, const float2* spec, const int* d_index, const int* r_index, int unit_scale,
+                       const float* pdirect, const float* pflip, ShiftParam* shiftp,
+                       int items) {
+    CorrSpecArgs ca{};
+    ca.spec = spec;
+    ca.d_index = d_index;
+    ca.r_index = r_index;
+    ca.out1 = c->work;
+    ca.out2 = c->work2;
+    ca.win = c->corrwin;
+    ca.unit_scale = unit_scale;
+    SPR_TRY2(corr_spec(c, ca, items));
+    return pick_shifts(c, pdirect, pflip, shiftp, items);
 }
 
 // ---------------------------------------------------------------------------
@@ -1423,11 +1450,12 @@ static int create_context(spr_ctx** out, int n, int capacity, int npat, const fl
         return cleanup_fail("hipMalloc row lists", e);
     if ((e = hipMalloc(&c->amp, np * npat * sizeof(float))) != hipSuccess) return cleanup_fail("hipMalloc amp", e);
     if ((e = hipMalloc(&c->amp_t, np * npat * sizeof(float))) != hipSuccess) return cleanup_fail("hipMalloc amp_t", e);
+    if ((e = hipMalloc(&c->corrwin, np * sizeof(float))) != hipSuccess) return cleanup_fail("hipMalloc corrwin", e);
     if ((e = hipMalloc(&c->tw, n * sizeof(float2))) != hipSuccess) return cleanup_fail("hipMalloc tw", e);
     if ((e = hipMalloc(&c->work2, np * capacity * sizeof(float2))) != hipSuccess)
         return cleanup_fail("hipMalloc work2", e);
     {
-        const int per = std::max(n / rows_per_wg(n), n / cols_per_wg(n));
+        const int per = std::max(n / rows_per_wg(n), n / std::min(cols_per_wg(n), aux_cols_per_wg(n)));
         c->partial_cap = (size_t)capacity * per * 2;
         if ((e = hipMalloc(&c->partial, c->partial_cap * sizeof(double))) != hipSuccess)
             return cleanup_fail("hipMalloc partial", e);
@@ -1501,6 +1529,7 @@ int spr_destroy(spr_ctx* c) {
     (void)hipFree(c->rowflags);
     (void)hipFree(c->amp);
     (void)hipFree(c->amp_t);
+    (void)hipFree(c->corrwin);
     (void)hipFree(c->amp_of);
     for (float2* t : c->twtab) (void)hipFree(t);
     (void)hipFree(c->tw);
@@ -1855,29 +1884,35 @@ int spr_align(spr_ctx* c, const float* ref_rho, float minr, float maxr, const fl
     if (P <= 0) return SPR_OK;
     const size_t np = (size_t)c->n * c->n;
     SPR_HIP(c, hipSetDevice(c->device));
-    SPR_TRY(ensure(c, c->spec, (P + 1) * np * sizeof(float2)));
+    SPR_TRY(ensure(c, c->spec, np * sizeof(float2)));   // the reference's spectrum
     SPR_TRY(ensure(c, c->fieldbuf, np * sizeof(float2)));
     SPR_TRY(ensure(c, c->supp2, (size_t)c->cap * np));
     SPR_TRY(ensure(c, c->shiftp, (size_t)P * sizeof(ShiftParam)));
     SPR_TRY(ensure(c, c->xphase, 2 * (size_t)P * sizeof(float)));
-    SPR_TRY(ensure(c, c->xidx, 2 * (size_t)P * sizeof(int)));
-    std::vector<int> idx(2 * (size_t)P);
-    for (int i = 0; i < P; ++i) {
-        idx[i] = i;        // d: the individual's spectrum
-        idx[P + i] = P;    // r: the reference spectrum
-    }
     float2* spec = (float2*)c->spec.p;
     float* ph = (float*)c->xphase.p;
-    int* di = (int*)c->xidx.p;
     ShiftParam* sp = (ShiftParam*)c->shiftp.p;
     SPR_HIP(c, hipMemcpyAsync(c->fieldbuf.p, ref_rho, np * sizeof(float2), hipMemcpyHostToDevice, c->stream));
     SPR_HIP(c, hipMemcpyAsync(ph, phase_direct, P * sizeof(float), hipMemcpyHostToDevice, c->stream));
     SPR_HIP(c, hipMemcpyAsync(ph + P, phase_flip, P * sizeof(float), hipMemcpyHostToDevice, c->stream));
-    SPR_HIP(c, hipMemcpyAsync(di, idx.data(), idx.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
-    // set_ref_density and get_shift both unit-scale their spectra (normalize_ft_shift)
-    SPR_TRY(modulus_spectra(c, c->rho, nullptr, spec, P));
-    SPR_TRY(modulus_spectra(c, (const float2*)c->fieldbuf.p, nullptr, spec + (size_t)P * np, 1));
-    SPR_TRY(correlate_and_pick(c, spec, di, di + P, minr, maxr, 1, ph, ph + P, sp, P));
+    SPR_TRY(corr_window(c, minr, maxr));
+    // set_ref_density and get_shift both unit-scale their spectra
+    // (normalize_ft_shift): the reference's in a pass of its own, the individuals'
+    // in the column pass that correlates them with it.
+    AuxRowArgs ar = aux_row_args(c);
+    ar.src = (const float2*)c->fieldbuf.p;
+    ar.work = spec;
+    SPR_TRY(row_aux(c, AROW_ABS_FWD_RHO, ar, 1));
+    AuxColArgs ca = aux_col_args(c);
+    ca.f = spec;
+    SPR_TRY(col_aux(c, ACOL_FWD_UNIT, ca, 1));
+    SPR_TRY(row_aux(c, AROW_ABS_FWD_RHO, aux_row_args(c), P));
+    ca.f = c->work;
+    ca.ref = spec;
+    ca.win = c->corrwin;
+    ca.unit_scale = 1;
+    SPR_TRY(col_aux(c, ACOL_CORR, ca, P));
+    SPR_TRY(pick_shifts(c, ph, ph + P, sp, P));
     ReshiftArgs ra{};
     ra.src = c->rho;
     ra.ssupp = c->supp;
@@ -2083,12 +2118,13 @@ int spr_crossover(spr_ctx* c, int nchild, const spr_cross_desc* desc, const int3
     SPR_HIP(c, hipMemcpyAsync(c->fieldbuf.p, avg_rho, np * sizeof(float2), hipMemcpyHostToDevice, c->stream));
     SPR_HIP(c, hipMemcpyAsync(c->ampavg.p, amp_avg, np * sizeof(float), hipMemcpyHostToDevice, c->stream));
 
+    SPR_TRY(corr_window(c, minr, maxr));
     // prepare_parents: spectra FT(|rho|) of the population and of the average (not unit-scaled)
     SPR_TRY(modulus_spectra(c, c->rho, nullptr, spec, P));
     if (with_avg) SPR_TRY(modulus_spectra(c, (const float2*)c->fieldbuf.p, nullptr, spec + (size_t)P * np, 1));
     // reshift_parent of p0, p2, p3 (and the average) against p1
     for (int r = 0; r < (with_avg ? 4 : 3); ++r) {
-        SPR_TRY(correlate_and_pick(c, spec, dlist(I_D, r), dlist(I_R, r), minr, maxr, 0, dph + (size_t)r * 2 * K,
+        SPR_TRY(correlate_and_pick(c, spec, dlist(I_D, r), dlist(I_R, r), 0, dph + (size_t)r * 2 * K,
                                    dph + (size_t)r * 2 * K + K, sp, K));
         ReshiftArgs ra{};
         ra.src = r < 3 ? c->rho : (const float2*)c->fieldbuf.p;

@@ -26,12 +26,14 @@ def supports(n, disk):
     return s
 
 
-@pytest.mark.parametrize("n", [256, 384, 512, 768, 1024])
+@pytest.mark.parametrize("n", [64, 128, 256, 384, 512, 768, 1024])
 @pytest.mark.parametrize("alg,beta", [("HIO", 0.9), ("RAAR", 0.87), ("ER", 0.0)])
 def test_two_iterations_by_rows(hip, orc, n, alg, beta):
     amp, rho, disk = case(n, 4, seed=17)
     supp = supports(n, disk[0])
     be = hip.Backend(amp, capacity=4)
+    if n <= 128:
+        be.set_fused(1)     # on chip: wavefronts of eight (128^2) or sixteen (64^2) rows
     be.set_population(rho, supp)
     be.iterate(alg, 2, beta, 0.0)
     got, s = be.get_population()
