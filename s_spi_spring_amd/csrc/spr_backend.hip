@@ -579,9 +579,9 @@ int queue_blur_magnitude(spr_ctx* c, float sigma, bool want_max) {
 int queue_sw(spr_ctx* c, float sigma, float threshold) {
     if (c->P <= 0) return SPR_OK;
     SPR_TRY2(queue_blur_magnitude(c, sigma, true));
-    const size_t total = (size_t)c->n * c->n * c->P;
-    hipLaunchKernelGGL(k_cut_max, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, c->stream,
-                       (const float*)c->work2, (const unsigned*)c->maxbits, threshold, c->supp, c->n * c->n, c->P);
+    const int wgs = c->n * c->n / 1024;   // every supported size is a multiple of 64
+    hipLaunchKernelGGL(k_cut_max, dim3((unsigned)((size_t)wgs * c->P)), dim3(256), 0, c->stream,
+                       (const float4*)c->work2, (const unsigned*)c->maxbits, threshold, (uchar4*)c->supp, wgs);
     SPR_HIP(c, hipGetLastError());
     return SPR_OK;
 }
