@@ -966,8 +966,10 @@ int correlate_and_pick(spr_ctx* c, const float2* spec, const int* d_index, const
 // loss partial per workgroup.
 template <int N, int CV> int launch_col_loss_v(spr_ctx* c, LossArgs a, int items, bool want_loss) {
     using G = typename ColVariant<N, CV>::G;
-    if (G::TW_GLOBAL && !c->twtab[CV]) return fail(c, SPR_ERR_STATE, "twiddle table missing");
-    a.twtab = c->twtab[CV];
+    if constexpr (G::TW_GLOBAL) {
+        if (!c->twtab[CV]) return fail(c, SPR_ERR_STATE, "twiddle table missing");
+        a.twtab = c->twtab[CV];
+    }
     const dim3 grid((unsigned)((size_t)items * (N / G::C))), block(G::COL_THREADS);
     if (want_loss) hipLaunchKernelGGL((k_col_loss<N, CV, true>), grid, block, 0, c->stream, a);
     else hipLaunchKernelGGL((k_col_loss<N, CV, false>), grid, block, 0, c->stream, a);
@@ -1010,7 +1012,7 @@ template <int N> int launch_col_loss(spr_ctx* c, LossArgs a, int items, bool wan
                 break;
         }
     }
-    return launch_col_loss_v<N, 0>(c, a, items, want_loss);
+    return launch_col_loss_v<N, loss_variant<N>()>(c, a, items, want_loss);
 }
 // The loss pass with one loss partial per workgroup (n / cols_per_wg(n) per
 // field) in the default geometry, and the refinement steps' gradient pass

@@ -57,12 +57,20 @@ __attribute__((amdgpu_waves_per_eu((ColVariant<N, CV>::G::COL_WAVES_PER_EU)))) v
     float2 v[V];
     float Aq[V];
 #pragma unroll
-    for (int r = 0; r < V; ++r) {
-        v[r] = f[off + r * T * N];
-        Aq[r] = amp[off + r * T * N];
+    for (int r = 0; r < V; ++r) v[r] = f[off + r * T * N];
+    // With two workgroups of 16 wavefronts on a CU (64 registers) the amplitude, in
+    // the L2, is read after the transform.
+    constexpr bool AMP_EARLY = CV != LOSS_VARIANT;
+    if constexpr (AMP_EARLY) {
+#pragma unroll
+        for (int r = 0; r < V; ++r) Aq[r] = amp[off + r * T * N];
     }
     __syncthreads();
     fft_line_p<PL, +1>(v, acc, tw, t);
+    if constexpr (!AMP_EARLY) {
+#pragma unroll
+        for (int r = 0; r < V; ++r) Aq[r] = amp[off + r * T * N];
+    }
     double l[1] = {0.0};
 #pragma unroll
     for (int q = 0; q < V; ++q) {
@@ -83,13 +91,13 @@ __attribute__((amdgpu_waves_per_eu((ColVariant<N, CV>::G::COL_WAVES_PER_EU)))) v
         }
         v[q] = make_float2(v[q].x * w, v[q].y * w);
     }
+    fft_line_p<PL, -1>(v, acc, tw, t);
+#pragma unroll
+    for (int q = 0; q < V; ++q) f[off + q * T * N] = v[q];
     if constexpr (WANT_LOSS) {
         block_sum<1, NT>(l, red);
         if (tid == 0) a.partial[strip] = l[0];
     }
-    fft_line_p<PL, -1>(v, acc, tw, t);
-#pragma unroll
-    for (int q = 0; q < V; ++q) f[off + q * T * N] = v[q];
 }
 
 // Projection onto the supports: rho <- 0 outside each individual's support (the
