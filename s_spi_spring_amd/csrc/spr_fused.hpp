@@ -45,6 +45,7 @@ struct FusedArgs {
     float beta;
     float inv_nn;
     PhaseCut pc;
+    float inv_n;            // 1/N
 };
 
 template <int N, int MODE>
@@ -62,7 +63,7 @@ __global__ __launch_bounds__(N * (N / 16)) void k_iter_fused(FusedArgs a) {
     const int p = blockIdx.x;
     const size_t base = (size_t)p * N * N;
     // Row phase: row `row`, elements x = t + T*j.
-    const int t = tid % T;
+    int t = tid % T;
     const int row = tid / T;
     const RowAccT<SH> racc{lds + row * RS};
     // Element t + T*j of the row: since t < T and T divides 2^SH,
@@ -70,7 +71,7 @@ __global__ __launch_bounds__(N * (N / 16)) void k_iter_fused(FusedArgs a) {
     float2* const rp = lds + row * RS + t;
     // Column phase: column `col`, elements y = tc + T*j.
     const int lane = tid % 64;
-    const int tc = lane / LPW;
+    int tc = lane / LPW;
     const int col = (tid / 64) * LPW + lane % LPW;
     const ColAcc<RS> cacc{lds + col + (col >> SH)};
     // Amplitude at (y, x) = (tc + T j, col), from the transposed copy
@@ -89,21 +90,70 @@ __global__ __launch_bounds__(N * (N / 16)) void k_iter_fused(FusedArgs a) {
             sbits |= (s0[t + T * j] != 0 ? 1u : 0u) << j;
         }
     }
-    __syncthreads();   // twiddle table
+    // A wavefront none of whose rows meets the support (10 - 35 % of the rows do, so
+    // most are) keeps their state as its row transform: the update is linear there
+    // (HIO, RAAR) or zero (ER) and needs no row transform, half of its share of the
+    // iteration. 128^2 x 256, HIO 20: 270 -> 253 us (the
+    // column phases, the same for every wavefront, are half of the rest, and HIO and
+    // RAAR spill 52 - 60 bytes of registers at 128, the limit of 16 wavefronts).
+    // (With an empty support every row runs the general update, which keeps the signs
+    // of zero that the projection of a vanishing spectrum depends on.)
+    const int any = __syncthreads_or(sbits != 0);   // and the twiddle table
+    const int outside = any && __ballot(sbits != 0) == 0;
+    const float lin_p = MODE == ROW_HIO ? -(a.beta * a.inv_n) : (1.f - 2.f * a.beta) * a.inv_n;
 #pragma unroll
     for (int j = 0; j < V; ++j) v[j] = rn[j];
     fft_line_p<PL, +1, true>(v, racc, tw, t);
+    if (outside) {
+#pragma unroll
+        for (int j = 0; j < V; ++j) rn[j] = v[j];
+    }
 #pragma unroll
     for (int j = 0; j < V; ++j) rp[T * j + ((T * j) >> SH)] = v[j];
 
-    for (int it = 0;; ++it) {
+    if (outside) {
+        // Column phases and, in place of the row transforms, the linear update.
+        for (int it = 0; it < a.niter; ++it) {
+            __syncthreads();
+            asm volatile("" : "+v"(t), "+v"(tc));
+            // column phase: colIFFT(P_M(colFFT(.)))
+#pragma unroll
+            for (int j = 0; j < V; ++j) v[j] = cacc.template ldk<T>(tc, j);
+            fft_line_p<PL, +1, true>(v, cacc, tw, tc);
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                if (j % 8 == 0) asm volatile("" ::: "memory");   // amplitudes eight at a time
+                v[j] = project_modulus(v[j], at[aoff + T * j]);
+            }
+            fft_line_p<PL, -1, true>(v, cacc, tw, tc);
+#pragma unroll
+            for (int j = 0; j < V; ++j) cacc.template stk<T>(tc, j, v[j]);
+            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                float2* const z = rp + T * j + ((T * j) >> SH);
+                const float2 pr = *z;
+                float2 o = make_float2(0.f, 0.f);
+                if constexpr (MODE == ROW_HIO) o = make_float2(rn[j].x + lin_p * pr.x, rn[j].y + lin_p * pr.y);
+                if constexpr (MODE == ROW_RAAR)
+                    o = make_float2(a.beta * rn[j].x + lin_p * pr.x, a.beta * rn[j].y + lin_p * pr.y);
+                rn[j] = o;
+                *z = o;
+            }
+        }
+    }
+    for (int it = outside ? a.niter : 0;; ++it) {
         __syncthreads();
+        asm volatile("" : "+v"(t), "+v"(tc));
         // column phase: colIFFT(P_M(colFFT(.)))
 #pragma unroll
         for (int j = 0; j < V; ++j) v[j] = cacc.template ldk<T>(tc, j);
         fft_line_p<PL, +1, true>(v, cacc, tw, tc);
 #pragma unroll
-        for (int j = 0; j < V; ++j) v[j] = project_modulus(v[j], at[aoff + T * j]);
+        for (int j = 0; j < V; ++j) {
+            if (j % 8 == 0) asm volatile("" ::: "memory");   // amplitudes eight at a time
+            v[j] = project_modulus(v[j], at[aoff + T * j]);
+        }
         fft_line_p<PL, -1, true>(v, cacc, tw, tc);
 #pragma unroll
         for (int j = 0; j < V; ++j) cacc.template stk<T>(tc, j, v[j]);
