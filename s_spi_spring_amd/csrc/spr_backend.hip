@@ -56,6 +56,7 @@ struct spr_ctx {
     float2* work2 = nullptr;      // second half-transformed field per individual (correlations, |b|)
     uint8_t* supp = nullptr;
     uint32_t* sbits = nullptr;    // supports one bit per pixel, packed at the start of every iteration block
+    void* planbuf = nullptr;      // the allocation of corrwin and the next four
     // Rows that meet each support, made with sbits (SupportPlan in spr_kernels.hpp).
     int* rowcnt = nullptr;        // [cap]
     uint16_t* rowlist = nullptr;  // [cap][n]
@@ -66,7 +67,8 @@ struct spr_ctx {
     float* amp_t = nullptr;       // amp transposed (read along columns by the column pass)
     int npat = 1;                 // patterns sharing this handle (one amplitude each)
     int colvar = 0, rowvar = 0;   // variants of the column and row iteration passes
-    float2* twtab[MAX_VARIANTS] = {};  // global twiddle tables of the column variants that read one
+    float2* twbuf = nullptr;           // twiddle tables of the column variants
+    float2* twtab[MAX_VARIANTS] = {};  // each variant's, in twbuf
     size_t chunk_bytes = 0;       // iteration blocks run in chunks of this working set (0: whole population)
     int fused = -1;               // on-chip iteration blocks (N <= 128): -1 by population size, 0 never, 1 always
     int* amp_of = nullptr;        // slot -> pattern when npat > 1, else NULL
@@ -312,19 +314,29 @@ template <int N, int CV = 0> int launch_step(spr_ctx* c, const Step& st, int cnt
     }
 }
 
-// Global twiddle tables of every column variant of size N (read by the step
-// passes, and by the column passes of variants with TW_GLOBAL).
-template <int N, int CV = 0> int build_twtabs(spr_ctx* c) {
+// Twiddle tables of every column variant of size N (read by the step passes, and
+// by the column passes of variants with TW_GLOBAL), one after another in one
+// allocation.
+template <int N, int CV = 0> constexpr size_t twtab_entries() {
     if constexpr (CV < MAX_VARIANTS) {
+        size_t n = 0;
+        if constexpr (ColVariant<N, CV>::valid) n = TwTableP<typename ColVariant<N, CV>::G::PL>::SIZE;
+        return n + twtab_entries<N, CV + 1>();
+    }
+    return 0;
+}
+template <int N, int CV = 0> int build_twtabs(spr_ctx* c, size_t at = 0) {
+    if constexpr (CV < MAX_VARIANTS) {
+        if constexpr (CV == 0) SPR_HIP(c, hipMalloc(&c->twbuf, twtab_entries<N>() * sizeof(float2)));
         if constexpr (ColVariant<N, CV>::valid) {
             using G = typename ColVariant<N, CV>::G;
-            constexpr int SIZE = TwTableP<typename G::PL>::SIZE;
-            SPR_HIP(c, hipMalloc(&c->twtab[CV], SIZE * sizeof(float2)));
+            c->twtab[CV] = c->twbuf + at;
+            at += TwTableP<typename G::PL>::SIZE;
             hipLaunchKernelGGL((k_build_twtab<typename G::PL>), dim3(1), dim3(256), 0, c->stream, c->twtab[CV],
                                (const float2*)c->tw);
             SPR_HIP(c, hipGetLastError());
         }
-        return build_twtabs<N, CV + 1>(c);
+        return build_twtabs<N, CV + 1>(c, at);
     }
     return SPR_OK;
 }
@@ -1445,14 +1457,18 @@ static int create_context(spr_ctx** out, int n, int capacity, int npat, const fl
         return cleanup_fail("hipMalloc work", e);
     if ((e = hipMalloc(&c->supp, np * capacity)) != hipSuccess) return cleanup_fail("hipMalloc supp", e);
     if ((e = hipMalloc(&c->sbits, np / 8 * capacity)) != hipSuccess) return cleanup_fail("hipMalloc sbits", e);
-    if ((e = hipMalloc(&c->rowcnt, (size_t)capacity * sizeof(int))) != hipSuccess ||
-        (e = hipMalloc(&c->rowlist, (size_t)capacity * n * sizeof(uint16_t))) != hipSuccess ||
-        (e = hipMalloc(&c->colmask, (size_t)capacity * (n / 8) * sizeof(uint32_t))) != hipSuccess ||
-        (e = hipMalloc(&c->rowflags, (size_t)capacity * (n / 32) * sizeof(uint32_t))) != hipSuccess)
-        return cleanup_fail("hipMalloc row lists", e);
+    {   // 4-byte arrays first, the 2-byte row lists last
+        const size_t cap = (size_t)capacity, masks = cap * (n / 8), flags = cap * (n / 32);
+        if ((e = hipMalloc(&c->planbuf, (np + masks + flags + cap) * 4 + cap * n * sizeof(uint16_t))) != hipSuccess)
+            return cleanup_fail("hipMalloc row lists", e);
+        c->corrwin = (float*)c->planbuf;
+        c->colmask = (uint32_t*)(c->corrwin + np);
+        c->rowflags = c->colmask + masks;
+        c->rowcnt = (int*)(c->rowflags + flags);
+        c->rowlist = (uint16_t*)(c->rowcnt + cap);
+    }
     if ((e = hipMalloc(&c->amp, np * npat * sizeof(float))) != hipSuccess) return cleanup_fail("hipMalloc amp", e);
     if ((e = hipMalloc(&c->amp_t, np * npat * sizeof(float))) != hipSuccess) return cleanup_fail("hipMalloc amp_t", e);
-    if ((e = hipMalloc(&c->corrwin, np * sizeof(float))) != hipSuccess) return cleanup_fail("hipMalloc corrwin", e);
     if ((e = hipMalloc(&c->tw, n * sizeof(float2))) != hipSuccess) return cleanup_fail("hipMalloc tw", e);
     if ((e = hipMalloc(&c->work2, np * capacity * sizeof(float2))) != hipSuccess)
         return cleanup_fail("hipMalloc work2", e);
@@ -1525,15 +1541,11 @@ int spr_destroy(spr_ctx* c) {
     (void)hipFree(c->work);
     (void)hipFree(c->supp);
     (void)hipFree(c->sbits);
-    (void)hipFree(c->rowcnt);
-    (void)hipFree(c->rowlist);
-    (void)hipFree(c->colmask);
-    (void)hipFree(c->rowflags);
     (void)hipFree(c->amp);
     (void)hipFree(c->amp_t);
-    (void)hipFree(c->corrwin);
+    (void)hipFree(c->planbuf);
     (void)hipFree(c->amp_of);
-    for (float2* t : c->twtab) (void)hipFree(t);
+    (void)hipFree(c->twbuf);
     (void)hipFree(c->tw);
     (void)hipFree(c->work2);
     (void)hipFree(c->partial);
