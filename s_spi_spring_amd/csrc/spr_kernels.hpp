@@ -600,9 +600,9 @@ __global__ __launch_bounds__((RowVariant<N, RV>::G::ROW_THREADS)) void k_row(Row
 // Row update of an iteration that recomputes rho_n: the rows that meet the
 // support, RW at a time (the column pass, k_col_step, has updated the others).
 // Workgroup b takes field b % fields and group b / fields of its list; those past
-// the lists' ends come last and leave at once (workgroups that step through the
-// lists instead, twinned down to 4096, took the same time: 20 us at 512^2 x 64
-// with 22 % of the rows listed, against 60 us for the pass over every row).
+// the lists' ends come last and leave at once (4096 workgroups that step through
+// the lists instead took the same time: 20 us at 512^2 x 64 with 22 % of the rows
+// listed, against 60 us for the pass over every row).
 template <int N, int MODE, int RV>
 __global__ __launch_bounds__((RowVariant<N, RV>::G::ROW_THREADS)) void k_row_listed(RowArgs a, int fields) {
     using G = typename RowVariant<N, RV>::G;
