@@ -819,7 +819,7 @@ int queue_iterate_block(spr_ctx* c, int mode, int niter, const RowArgs& a0) {
 // LDS (spr_fused.hpp): one launch, HBM read at its start and written at its end.
 template <int N> int launch_fused(spr_ctx* c, int mode, int niter, const RowArgs& a) {
     if constexpr (fused_size<N>()) {
-        const FusedArgs f{a.rho, a.supp, c->amp_t, c->amp_of, c->tw, niter, a.beta, a.inv_nn, a.pc, a.inv_n};
+        const FusedArgs f{a.rho, a.supp, c->amp_t, c->amp_of, c->tw, niter, a.beta, a.inv_nn, a.pc};
         const dim3 grid((unsigned)c->P), block(N * (N / 16));
         switch (mode) {
             case ROW_ER: hipLaunchKernelGGL((k_iter_fused<N, ROW_ER>), grid, block, 0, c->stream, f); break;

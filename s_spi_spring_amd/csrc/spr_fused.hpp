@@ -45,7 +45,6 @@ struct FusedArgs {
     float beta;
     float inv_nn;
     PhaseCut pc;
-    float inv_n;            // 1/N
 };
 
 template <int N, int MODE>
@@ -63,7 +62,7 @@ __global__ __launch_bounds__(N * (N / 16)) void k_iter_fused(FusedArgs a) {
     const int p = blockIdx.x;
     const size_t base = (size_t)p * N * N;
     // Row phase: row `row`, elements x = t + T*j.
-    int t = tid % T;
+    const int t = tid % T;
     const int row = tid / T;
     const RowAccT<SH> racc{lds + row * RS};
     // Element t + T*j of the row: since t < T and T divides 2^SH,
@@ -71,7 +70,7 @@ __global__ __launch_bounds__(N * (N / 16)) void k_iter_fused(FusedArgs a) {
     float2* const rp = lds + row * RS + t;
     // Column phase: column `col`, elements y = tc + T*j.
     const int lane = tid % 64;
-    int tc = lane / LPW;
+    const int tc = lane / LPW;
     const int col = (tid / 64) * LPW + lane % LPW;
     const ColAcc<RS> cacc{lds + col + (col >> SH)};
     // Amplitude at (y, x) = (tc + T j, col), from the transposed copy
@@ -93,14 +92,15 @@ __global__ __launch_bounds__(N * (N / 16)) void k_iter_fused(FusedArgs a) {
     // A wavefront none of whose rows meets the support (10 - 35 % of the rows do, so
     // most are) keeps their state as its row transform: the update is linear there
     // (HIO, RAAR) or zero (ER) and needs no row transform, half of its share of the
-    // iteration. 128^2 x 256, HIO 20: 270 -> 253 us (the
-    // column phases, the same for every wavefront, are half of the rest, and HIO and
-    // RAAR spill 52 - 60 bytes of registers at 128, the limit of 16 wavefronts).
+    // iteration (the column phases, the same for every wavefront, are half of the
+    // rest). All wavefronts run one loop, with its barriers and the update in common,
+    // and `outside`, uniform over a wavefront, only skips its two row transforms: with
+    // a loop of its own for those wavefronts the kernel spilled 52 - 60 bytes of
+    // registers at 128, the limit of 16 wavefronts, and 12 as it is.
     // (With an empty support every row runs the general update, which keeps the signs
     // of zero that the projection of a vanishing spectrum depends on.)
     const int any = __syncthreads_or(sbits != 0);   // and the twiddle table
-    const int outside = any && __ballot(sbits != 0) == 0;
-    const float lin_p = MODE == ROW_HIO ? -(a.beta * a.inv_n) : (1.f - 2.f * a.beta) * a.inv_n;
+    const int outside = __builtin_amdgcn_readfirstlane(any && __ballot(sbits != 0) == 0);
 #pragma unroll
     for (int j = 0; j < V; ++j) v[j] = rn[j];
     fft_line_p<PL, +1, true>(v, racc, tw, t);
@@ -111,49 +111,14 @@ __global__ __launch_bounds__(N * (N / 16)) void k_iter_fused(FusedArgs a) {
 #pragma unroll
     for (int j = 0; j < V; ++j) rp[T * j + ((T * j) >> SH)] = v[j];
 
-    if (outside) {
-        // Column phases and, in place of the row transforms, the linear update.
-        for (int it = 0; it < a.niter; ++it) {
-            __syncthreads();
-            asm volatile("" : "+v"(t), "+v"(tc));
-            // column phase: colIFFT(P_M(colFFT(.)))
-#pragma unroll
-            for (int j = 0; j < V; ++j) v[j] = cacc.template ldk<T>(tc, j);
-            fft_line_p<PL, +1, true>(v, cacc, tw, tc);
-#pragma unroll
-            for (int j = 0; j < V; ++j) {
-                if (j % 8 == 0) asm volatile("" ::: "memory");   // amplitudes eight at a time
-                v[j] = project_modulus(v[j], at[aoff + T * j]);
-            }
-            fft_line_p<PL, -1, true>(v, cacc, tw, tc);
-#pragma unroll
-            for (int j = 0; j < V; ++j) cacc.template stk<T>(tc, j, v[j]);
-            __syncthreads();
-#pragma unroll
-            for (int j = 0; j < V; ++j) {
-                float2* const z = rp + T * j + ((T * j) >> SH);
-                const float2 pr = *z;
-                float2 o = make_float2(0.f, 0.f);
-                if constexpr (MODE == ROW_HIO) o = make_float2(rn[j].x + lin_p * pr.x, rn[j].y + lin_p * pr.y);
-                if constexpr (MODE == ROW_RAAR)
-                    o = make_float2(a.beta * rn[j].x + lin_p * pr.x, a.beta * rn[j].y + lin_p * pr.y);
-                rn[j] = o;
-                *z = o;
-            }
-        }
-    }
-    for (int it = outside ? a.niter : 0;; ++it) {
+    for (int it = 0;; ++it) {
         __syncthreads();
-        asm volatile("" : "+v"(t), "+v"(tc));
         // column phase: colIFFT(P_M(colFFT(.)))
 #pragma unroll
         for (int j = 0; j < V; ++j) v[j] = cacc.template ldk<T>(tc, j);
         fft_line_p<PL, +1, true>(v, cacc, tw, tc);
 #pragma unroll
-        for (int j = 0; j < V; ++j) {
-            if (j % 8 == 0) asm volatile("" ::: "memory");   // amplitudes eight at a time
-            v[j] = project_modulus(v[j], at[aoff + T * j]);
-        }
+        for (int j = 0; j < V; ++j) v[j] = project_modulus(v[j], at[aoff + T * j]);
         fft_line_p<PL, -1, true>(v, cacc, tw, tc);
 #pragma unroll
         for (int j = 0; j < V; ++j) cacc.template stk<T>(tc, j, v[j]);
@@ -161,7 +126,12 @@ __global__ __launch_bounds__(N * (N / 16)) void k_iter_fused(FusedArgs a) {
         // row phase: rho' = rowIFFT(.)/N^2
 #pragma unroll
         for (int j = 0; j < V; ++j) v[j] = rp[T * j + ((T * j) >> SH)];
-        fft_line_p<PL, -1, true>(v, racc, tw, t);
+        if (!outside || it == a.niter) {
+            fft_line_p<PL, -1, true>(v, racc, tw, t);
+        } else {   // v / N^2 then is the row transform of rho'
+#pragma unroll
+            for (int j = 0; j < V; ++j) v[j] = make_float2(v[j].x * N, v[j].y * N);
+        }
         if (it == a.niter) {   // the trailing projection: rho <- rho'
             float2* __restrict__ r0 = a.rho + base + (size_t)row * N;
 #pragma unroll
@@ -193,7 +163,7 @@ __global__ __launch_bounds__(N * (N / 16)) void k_iter_fused(FusedArgs a) {
             rn[j] = o;
             v[j] = o;
         }
-        fft_line_p<PL, +1, true>(v, racc, tw, t);
+        if (!outside) fft_line_p<PL, +1, true>(v, racc, tw, t);
 #pragma unroll
         for (int j = 0; j < V; ++j) rp[T * j + ((T * j) >> SH)] = v[j];
     }
