@@ -284,9 +284,11 @@ template <int N, int CV> int launch_step_v(spr_ctx* c, const Step& st, int cnt, 
     if constexpr (has_recompute<N>()) {
         using G = typename ColVariant<N, CV>::G;
         if (!c->twtab[CV]) return fail(c, SPR_ERR_STATE, "twiddle table missing");
+        // Half-width strips while each of them finds a CU of its own.
+        const int narrow = narrow_strips<N, G>() && (size_t)cnt * (N / G::C) <= 128 ? 1 : 0;
         const StepArgs a{st.f, st.proj, c->amp, c->amp_of ? c->amp_of + first : nullptr, c->twtab[CV],
-                         c->colmask + (size_t)first * G::T, st.lin_w, st.lin_p, st.all_rows};
-        const dim3 grid((unsigned)((size_t)cnt * (N / G::C))), block(G::COL_THREADS);
+                         c->colmask + (size_t)first * G::T, st.lin_w, st.lin_p, st.all_rows, narrow};
+        const dim3 grid((unsigned)((size_t)cnt * (N / G::C) << narrow)), block(G::COL_THREADS >> narrow);
         switch (st.mode) {
             case STEP_LIN: hipLaunchKernelGGL((k_col_step<N, STEP_LIN, CV>), grid, block, 0, s, a); break;
             case STEP_ER: hipLaunchKernelGGL((k_col_step<N, STEP_ER, CV>), grid, block, 0, s, a); break;
@@ -302,11 +304,7 @@ template <int N, int CV> int launch_step_v(spr_ctx* c, const Step& st, int cnt, 
 template <int N, int CV = 0> int launch_step(spr_ctx* c, const Step& st, int cnt, hipStream_t s, int first) {
     if constexpr (CV < MAX_VARIANTS) {
         if constexpr (ColVariant<N, CV>::valid) {
-            if (c->colvar == CV) {
-                constexpr int CN = narrow_variant<N, CV>();
-                if (CN != CV && cnt * (N / ColVariant<N, CV>::G::C) < 256) return launch_step_v<N, CN>(c, st, cnt, s, first);
-                return launch_step_v<N, CV>(c, st, cnt, s, first);
-            }
+            if (c->colvar == CV) return launch_step_v<N, CV>(c, st, cnt, s, first);
         }
         return launch_step<N, CV + 1>(c, st, cnt, s, first);
     } else {

@@ -211,18 +211,6 @@ SPR_ROW_VARIANT(2048, 5, Plan<2048, 16, 16, 8, 16>, 0, 256, -1, 1, 0, 4, 0, 0, 1
 #undef SPR_COL_VARIANT
 #undef SPR_ROW_VARIANT
 
-// The column variant that k_col_step takes in place of CV while CV's strips leave
-// CUs without a workgroup: the same plan in tiles half as wide. At 512^2 x 1
-// (64 or 128 workgroups on 256 CUs) an iteration takes 11.1 instead of 12.2 us,
-// at 1024^2 x 1 17.8 instead of 19.0, at 384^2 x 1 13.7 instead of 14.2; from 256
-// workgroups on the wide tiles are even or ahead (512^2 x 4: 13.6 against 14.3).
-template <int N, int CV> constexpr int narrow_variant() {
-    if constexpr (N == 384 && CV == 1) return 3;
-    else if constexpr (N == 512 && CV == 1) return 7;
-    else if constexpr (N == 1024 && CV == 6) return 7;
-    else return CV;
-}
-
 // The column variant of the plain projection (k_col) in place of CV: the same plan
 // in the layout that pass runs best in, where it is not the step pass's. 512^2 x
 // 64: 52 us in the skewed tile, 60 in the padded one.
@@ -731,6 +719,17 @@ template <int N, int C = Geo<N>::C> __device__ __forceinline__ int col_strip(int
     }
 }
 
+// The same for strips of 2^lc columns, lc known at the launch.
+template <int N> __device__ __forceinline__ int col_strip(int b, int lc) {
+    if constexpr (SPR_COL_XCD == 0) {
+        return b;
+    } else {
+        const int lg = lc < 4 ? 4 - lc : 0;     // log2 of the strips per 128-byte line
+        const int j = b & ((8 << lg) - 1);
+        return (b - j) + ((j & 7) << lg) + (j >> 3);
+    }
+}
+
 // Column pass over C adjacent columns of one field. Global memory is read and
 // written as rows of C consecutive values (coalesced); the C columns' transforms
 // exchange data through a padded LDS tile with workgroup barriers. With
@@ -828,7 +827,19 @@ struct StepArgs {
     const uint32_t* colmask;  // [fields][N/V] row masks of k_pack_support
     float lin_w, lin_p;       // STEP_LIN: f <- lin_w f + lin_p projected outside the support
     int all_rows;             // STEP_ER*: rho_n is any density (the first pass of a block)
+    int narrow;               // 1: strips of C/2 columns (narrow_strips), 0: of C
 };
+
+constexpr int log2i(int x) { return x > 1 ? 1 + log2i(x / 2) : 0; }
+// Whether a field's strips of c columns fill col_strip's chunks (whole lines of 128
+// bytes, eight at a time), so that the strips of a field stay its own.
+constexpr bool whole_chunks(int n, int c) { return c >= 16 || (n / c) % (8 * (16 / c)) == 0; }
+// Whether k_col_step is also launched with strips of half its tile's columns: whole
+// wavefronts, at least four columns (32 bytes of a row), and grids of which one
+// field leaves most CUs without a strip of C.
+template <int N, class G> constexpr bool narrow_strips() {
+    return N <= 512 && G::C >= 8 && G::COL_THREADS / 2 % 64 == 0 && whole_chunks(N, G::C / 2);
+}
 
 // One field of N*N elements of E bytes as a raw buffer: addresses are a 32-bit
 // per-thread offset plus a scalar one, so the V rows of a thread cost no address
@@ -866,6 +877,16 @@ __device__ __forceinline__ int row_offset(int voff, uint32_t off_rows, int q) {
 // B/px for the pass, as for the plain projection, and the row pass (24 B/px and
 // two or three transforms) visits only the rows that meet the support, 10 - 45 %
 // of them for objects on an oversampled grid.
+// The strip's width is the launch's: C columns, or C/2 while that gives every strip
+// a CU of its own (at most 128 strips of C for 256 CUs). us per RAAR iteration, a
+// quarter of the rows listed, wide / narrow: 256^2 x 4 11.2 / 11.0, x 7 11.6 / 12.2;
+// 384^2 x 2 16.1 / 15.3, x 4 16.6 / 16.7; 512^2 x 1 13.2 / 12.2, x 2 13.7 / 12.8,
+// x 3 14.3 / 14.7; 768^2 x 1 19.1 / 19.3; 1024^2 x 1 20.9 / 20.4, but the width as
+// a variable costs that kernel 3 % of its time at every population.
+// Both widths run the same instructions on every column, in the tile laid out for
+// C, so that a column's values do not depend on which individuals share its
+// launch: a kernel compiled for the narrower tile contracts multiply-adds
+// differently, and at 384^2 gave other bits.
 template <int N, int MODE, int CV>
 __global__ __launch_bounds__((ColVariant<N, CV>::G::COL_THREADS))
 __attribute__((amdgpu_waves_per_eu((ColVariant<N, CV>::G::COL_WAVES_PER_EU)))) void k_col_step(StepArgs a) {
@@ -874,19 +895,23 @@ __attribute__((amdgpu_waves_per_eu((ColVariant<N, CV>::G::COL_WAVES_PER_EU)))) v
     constexpr int V = G::V, T = G::T, C = G::C;
     __shared__ float2 twl[G::TW_GLOBAL ? 1 : TwTableP<PL>::SIZE];
     __shared__ float2 lds[G::COL_TILE];
+    static_assert((C & (C - 1)) == 0 && whole_chunks(N, C), "strips fill the chunks of col_strip");
+    const int narrow = narrow_strips<N, G>() ? a.narrow : 0;
+    const int lc = log2i(C) - narrow;
     const int tid = threadIdx.x;
-    const int c = tid % C;
-    const int t = tid / C;
+    const int c = tid & ((1 << lc) - 1);
+    const int t = tid >> lc;
+    __builtin_assume(t < T);
     constexpr int TILES = N / C;
-    const int strip = col_strip<N, C>(blockIdx.x);
-    const int p = strip / TILES;
-    const int x0 = (strip % TILES) * C;
+    const int strip = col_strip<N>(blockIdx.x, lc);
+    const int p = (strip >> narrow) / TILES;
+    const int x0 = (strip - p * (TILES << narrow)) << lc;
     const uint32_t off_rows = ~a.colmask[(size_t)p * T + t];
     const float2* tw = twl;
     if constexpr (G::TW_GLOBAL) {
         tw = a.twtab;
     } else {
-        for (int e = tid; e < TwTableP<PL>::SIZE; e += G::COL_THREADS) twl[e] = a.twtab[e];
+        for (int e = tid; e < TwTableP<PL>::SIZE; e += T << lc) twl[e] = a.twtab[e];
     }
     const __amdgpu_buffer_rsrc_t bf = field_buffer<N, 8>(a.f + (size_t)p * N * N);
     const __amdgpu_buffer_rsrc_t ba = field_buffer<N, 4>(a.amp + amp_offset<N>(a.amp_of, p));
