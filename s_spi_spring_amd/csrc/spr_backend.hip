@@ -67,6 +67,7 @@ struct spr_ctx {
     float* amp_t = nullptr;       // amp transposed (read along columns by the column pass)
     int npat = 1;                 // patterns sharing this handle (one amplitude each)
     int colvar = 0, rowvar = 0;   // variants of the column and row iteration passes
+    bool exact = false;           // chosen by the caller or the autotuner: the plain projection runs colvar itself
     float2* twbuf = nullptr;           // twiddle tables of the column variants
     float2* twtab[MAX_VARIANTS] = {};  // each variant's, in twbuf
     size_t chunk_bytes = 0;       // iteration blocks run in chunks of this working set (0: whole population)
@@ -339,15 +340,27 @@ template <int N, int CV = 0> int build_twtabs(spr_ctx* c, size_t at = 0) {
     return SPR_OK;
 }
 
+// Column variant of the plain projection: the handle's, or, where the handle runs
+// the compiled choice, the one plain_variant names beside it.
+template <int N, int CV = 0> int plain_colvar(const spr_ctx* c) {
+    if (c->exact) return c->colvar;
+    if constexpr (CV < MAX_VARIANTS) return c->colvar == CV ? plain_variant<N, CV>() : plain_colvar<N, CV + 1>(c);
+    return c->colvar;
+}
 template <int N, int CV = 0> int launch_col(spr_ctx* c, int mode, float2* f, int cnt, hipStream_t s, int first) {
     if (mode != COL_PROJ) return launch_col_v<N, 0>(c, mode, f, cnt, s, first);
     if constexpr (CV < MAX_VARIANTS) {
         if constexpr (ColVariant<N, CV>::valid)
-            if (c->colvar == CV) return launch_col_v<N, plain_variant<N, CV>()>(c, mode, f, cnt, s, first);
+            if (plain_colvar<N>(c) == CV) return launch_col_v<N, CV>(c, mode, f, cnt, s, first);
         return launch_col<N, CV + 1>(c, mode, f, cnt, s, first);
     } else {
         return fail(c, SPR_ERR_ARG, "bad column variant");
     }
+}
+
+template <int N> int plain_colvar_n(spr_ctx* c, int* col) {
+    *col = plain_colvar<N>(c);
+    return SPR_OK;
 }
 
 // Grid sizes with compiled kernels (RadixPlan in spr_fft.hpp).
@@ -1152,6 +1165,7 @@ int final_loss(spr_ctx* c, int kind, float eps, double* loss) {
 // ---------------------------------------------------------------------------
 struct VariantPair {
     int col = 0, row = 0;
+    bool exact = false;    // chosen at run time, not from the compiled table
 };
 std::mutex g_variant_mu;
 std::map<int, VariantPair> g_variant;   // sizes whose default differs from the compiled table
@@ -1192,7 +1206,6 @@ VariantPair default_variants(int n) {
     return v;
 }
 
-// Mean duration (ms) of `reps` launches of one pass in the handle's current variant.
 // Average time of one iteration (column pass, then RAAR row pass) with the
 // handle's current variants. Timing whole iterations, not one pass repeated,
 // keeps the caches as the iteration leaves them: a pass that reads a table from
@@ -1242,8 +1255,7 @@ int autotune(spr_ctx* c, int reps, float* col_ms, float* row_ms) {
     RowArgs ra = row_args(c);
     ra.beta = 0.87f;
     ra.pc = cut_raar(0.f);
-    const VariantPair keep{c->colvar, c->rowvar};
-    c->rowvar = 0;
+    const VariantPair keep{c->colvar, c->rowvar, c->exact};
     hipEvent_t e0 = nullptr, e1 = nullptr;
     SPR_HIP(c, hipEventCreate(&e0));
     if (hipEventCreate(&e1) != hipSuccess) {
@@ -1263,7 +1275,8 @@ int autotune(spr_ctx* c, int reps, float* col_ms, float* row_ms) {
     float tc[MAX_VARIANTS] = {}, tr[MAX_VARIANTS] = {};
     int rc = SPR_OK;
     VariantPair best;
-    c->rowvar = keep.row;
+    best.exact = true;
+    c->exact = true;   // every variant is timed as itself
     for (int v = 0; v < nc && rc == SPR_OK; ++v) {
         c->colvar = v;
         rc = time_iteration(c, ra, reps, e0, e1, &tc[v]);
@@ -1282,6 +1295,7 @@ int autotune(spr_ctx* c, int reps, float* col_ms, float* row_ms) {
     if (rc != SPR_OK) {
         c->colvar = keep.col;
         c->rowvar = keep.row;
+        c->exact = keep.exact;
         return rc;
     }
     c->colvar = best.col;
@@ -1431,6 +1445,7 @@ static int create_context(spr_ctx** out, int n, int capacity, int npat, const fl
         const VariantPair v = default_variants(n);
         c->colvar = v.col;
         c->rowvar = v.row;
+        c->exact = v.exact;
     }
     const size_t np = (size_t)n * n;
     auto cleanup_fail = [&](const char* what, hipError_t e) {
@@ -2372,7 +2387,7 @@ int spr_set_default_variants(int n, int col, int row) {
     if (variant_counts(n, &nc, &nr) != SPR_OK) return fail(nullptr, SPR_ERR_ARG, "unsupported grid size");
     if (col < 0 || col >= nc || row < 0 || row >= nr) return fail(nullptr, SPR_ERR_ARG, "variant out of range");
     std::lock_guard<std::mutex> lk(g_variant_mu);
-    g_variant[n] = VariantPair{col, row};
+    g_variant[n] = VariantPair{col, row, true};
     return SPR_OK;
 }
 
@@ -2384,6 +2399,7 @@ int spr_set_variants(spr_ctx* c, int col, int row) {
     SPR_HIP(c, hipStreamSynchronize(c->stream));
     c->colvar = col;
     c->rowvar = row;
+    c->exact = true;
     return SPR_OK;
 }
 
@@ -2392,6 +2408,11 @@ int spr_get_variants(spr_ctx* c, int* col, int* row) {
     if (col) *col = c->colvar;
     if (row) *row = c->rowvar;
     return SPR_OK;
+}
+
+int spr_get_plain_variant(spr_ctx* c, int* col) {
+    if (!c || !col) return fail(c, SPR_ERR_ARG, "NULL argument");
+    SPR_DISPATCH_N(c, plain_colvar_n, c, col);
 }
 
 int spr_set_chunk(spr_ctx* c, long long bytes) {

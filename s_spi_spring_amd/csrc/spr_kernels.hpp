@@ -211,9 +211,9 @@ SPR_ROW_VARIANT(2048, 5, Plan<2048, 16, 16, 8, 16>, 0, 256, -1, 1, 0, 4, 0, 0, 1
 #undef SPR_COL_VARIANT
 #undef SPR_ROW_VARIANT
 
-// The column variant of the plain projection (k_col) in place of CV: the same plan
-// in the layout that pass runs best in, where it is not the step pass's. 512^2 x
-// 64: 52 us in the skewed tile, 60 in the padded one.
+// The column variant of the plain projection (k_col) where CV is the compiled choice
+// of the step pass: the same plan in the layout that pass runs best in. 512^2 x 64:
+// 52 us in the skewed tile, 60 in the padded one.
 template <int N, int CV> constexpr int plain_variant() { return N == 512 && CV == 1 ? 6 : CV; }
 
 constexpr int MAX_VARIANTS = 8;
