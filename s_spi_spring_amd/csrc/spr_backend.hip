@@ -1009,40 +1009,23 @@ template <int N, int CV> constexpr bool same_plan_variant() {
     }
     return false;
 }
-template <int N> int launch_col_loss(spr_ctx* c, LossArgs a, int items, bool want_loss) {
-    if (!want_loss) {
-        switch (c->colvar) {
-            case 1:
-                if constexpr (same_plan_variant<N, 1>()) return launch_col_loss_v<N, 1>(c, a, items, false);
-                break;
-            case 2:
-                if constexpr (same_plan_variant<N, 2>()) return launch_col_loss_v<N, 2>(c, a, items, false);
-                break;
-            case 3:
-                if constexpr (same_plan_variant<N, 3>()) return launch_col_loss_v<N, 3>(c, a, items, false);
-                break;
-            case 4:
-                if constexpr (same_plan_variant<N, 4>()) return launch_col_loss_v<N, 4>(c, a, items, false);
-                break;
-            case 5:
-                if constexpr (same_plan_variant<N, 5>()) return launch_col_loss_v<N, 5>(c, a, items, false);
-                break;
-            case 6:
-                if constexpr (same_plan_variant<N, 6>()) return launch_col_loss_v<N, 6>(c, a, items, false);
-                break;
-            case 7:
-                if constexpr (same_plan_variant<N, 7>()) return launch_col_loss_v<N, 7>(c, a, items, false);
-                break;
-        }
+template <int N, int CV = 0> int launch_col_grad(spr_ctx* c, const LossArgs& a, int items) {
+    if constexpr (CV < MAX_VARIANTS) {
+        if constexpr (same_plan_variant<N, CV>())
+            if (c->colvar == CV) return launch_col_loss_v<N, CV>(c, a, items, false);
+        return launch_col_grad<N, CV + 1>(c, a, items);
     }
-    return launch_col_loss_v<N, loss_variant<N>()>(c, a, items, want_loss);
+    return launch_col_loss_v<N, 0>(c, a, items, false);
+}
+template <int N> int launch_col_loss(spr_ctx* c, const LossArgs& a, int items, bool want_loss) {
+    if (!want_loss) return launch_col_grad<N>(c, a, items);
+    return launch_col_loss_v<N, 0>(c, a, items, true);
 }
 // The loss pass with one loss partial per workgroup (n / cols_per_wg(n) per
 // field) in the default geometry, and the refinement steps' gradient pass
 // without partials, in the handle's column variant when that variant holds the
-// default radix plan (the same gradients as spr_loss_grad, bit for bit), else
-// in the default geometry too (at 1024^2 the radix-16 variants measured no
-// faster for this pass: 0.577 against 0.575 ms per refinement step).
+// default radix plan (the same gradients as spr_loss_grad, bit for bit), else in the default geometry too (at 1024^2 the radix-16 variants
+// measured no faster for this pass: 0.577 against 0.575 ms per refinement step).
 int col_loss(spr_ctx* c, const LossArgs& a, int items) { SPR_DISPATCH_N(c, launch_col_loss, c, a, items, true); }
 int col_loss_step(spr_ctx* c, const LossArgs& a, int items) { SPR_DISPATCH_N(c, launch_col_loss, c, a, items, false); }
 

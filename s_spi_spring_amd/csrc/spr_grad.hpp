@@ -28,20 +28,31 @@ struct LossArgs {
     const float2* twtab; // the plan's twiddle table in global memory (column variants with TW_GLOBAL)
 };
 
+// Waves per SIMD of the loss passes: the column passes', but two workgroups on a CU
+// where only the 512 bytes those allow for keep it to one: at 1024^2, where the
+// tile and the twiddle table are 81 856 bytes and the 16 wavefronts of a workgroup
+// fit twice with 64 registers. Left to itself the allocation took 64 or 65: a launch
+// of 16 fields 95 or 133 us (the gradient alone); with the loss 134 us in one
+// workgroup, 106 in two, its sums reduced in the tile.
+template <class G> constexpr int loss_waves() {
+    constexpr int bytes = (G::COL_TILE + (G::TW_GLOBAL ? 0 : TwTableP<typename G::PL>::SIZE)) * 8;
+    return G::COL_WG == 1 && 2 * bytes <= 160 * 1024 && 2 * G::COL_THREADS <= 2048 ? 2 * G::COL_THREADS / 256
+                                                                                   : G::COL_WAVES_PER_EU;
+}
+
 // Column pass of the loss in the geometry of column variant CV (the tile
 // layouts of the projection pass). WANT_LOSS: one loss partial per workgroup
 // into a.partial[strip] (summed in double); without it the pass computes only
 // the weighted spectrum (the refinement steps, whose losses are not read).
 template <int N, int CV = 0, bool WANT_LOSS = true>
 __global__ __launch_bounds__((ColVariant<N, CV>::G::COL_THREADS))
-__attribute__((amdgpu_waves_per_eu((ColVariant<N, CV>::G::COL_WAVES_PER_EU)))) void k_col_loss(LossArgs a) {
+__attribute__((amdgpu_waves_per_eu((loss_waves<typename ColVariant<N, CV>::G>())))) void k_col_loss(LossArgs a) {
     using G = typename ColVariant<N, CV>::G;
     using PL = typename G::PL;
     constexpr int V = G::V, T = G::T, C = G::C, NT = G::COL_THREADS, TILES = N / C;
     static_assert(!G::COL_WAVE, "loss passes use LDS tiles of rows");
     __shared__ float2 twl[G::TW_GLOBAL ? 1 : TwTableP<PL>::SIZE];
     __shared__ float2 lds[G::COL_TILE];
-    __shared__ double red[WANT_LOSS ? 4 * (NT / 64) : 1];
     const int tid = threadIdx.x, c = tid % C, t = tid / C;
     const float2* tw = twl;
     if constexpr (G::TW_GLOBAL) tw = a.twtab;
@@ -57,20 +68,12 @@ __attribute__((amdgpu_waves_per_eu((ColVariant<N, CV>::G::COL_WAVES_PER_EU)))) v
     float2 v[V];
     float Aq[V];
 #pragma unroll
-    for (int r = 0; r < V; ++r) v[r] = f[off + r * T * N];
-    // With two workgroups of 16 wavefronts on a CU (64 registers) the amplitude, in
-    // the L2, is read after the transform.
-    constexpr bool AMP_EARLY = CV != LOSS_VARIANT;
-    if constexpr (AMP_EARLY) {
-#pragma unroll
-        for (int r = 0; r < V; ++r) Aq[r] = amp[off + r * T * N];
+    for (int r = 0; r < V; ++r) {
+        v[r] = f[off + r * T * N];
+        Aq[r] = amp[off + r * T * N];
     }
     __syncthreads();
     fft_line_p<PL, +1>(v, acc, tw, t);
-    if constexpr (!AMP_EARLY) {
-#pragma unroll
-        for (int r = 0; r < V; ++r) Aq[r] = amp[off + r * T * N];
-    }
     double l[1] = {0.0};
 #pragma unroll
     for (int q = 0; q < V; ++q) {
@@ -95,7 +98,7 @@ __attribute__((amdgpu_waves_per_eu((ColVariant<N, CV>::G::COL_WAVES_PER_EU)))) v
 #pragma unroll
     for (int q = 0; q < V; ++q) f[off + q * T * N] = v[q];
     if constexpr (WANT_LOSS) {
-        block_sum<1, NT>(l, red);
+        block_sum<1, NT>(l, reinterpret_cast<double*>(lds));   // the last transform leaves the tile free
         if (tid == 0) a.partial[strip] = l[0];
     }
 }

@@ -168,12 +168,6 @@ SPR_COL_VARIANT(512, 7, RadixPlan<512>, 4, 256, -1, 0, 0, 3, 2, 5)
 SPR_COL_VARIANT(768, 1, RadixPlan<768>, 4, 256, -1, 1, 0, 3, 2, 3)
 SPR_COL_VARIANT(768, 6, RadixPlan<768>, 4, 256, -1, 0, 0, 3, 2)
 SPR_COL_VARIANT(1024, 7, Plan<1024, 16, 16, 8, 8>, 4, 256, -1, 0, 0, 3, 4, 3)
-// The loss pass's own tile at 1024^2 (outside the autotuner's range): the default
-// plan, strip and partials, in a tile without row padding, so that with its
-// reduction two workgroups fit on a CU (78 KB; 82 KB in the default tile, one).
-constexpr int LOSS_VARIANT = 8;
-SPR_COL_VARIANT(1024, 8, RadixPlan<1024>, 8, 256, -1, 0, 0, 3, 4)
-template <int N> constexpr int loss_variant() { return N == 1024 ? LOSS_VARIANT : 0; }
 // row variants: plan, -, threads per workgroup, prefetch mode
 SPR_ROW_VARIANT(256, 1, RadixPlan<256>, 0, 512)
 SPR_ROW_VARIANT(384, 1, RadixPlan<384>, 0, 512)
