@@ -1012,7 +1012,7 @@ template <int N, int CV> constexpr bool same_plan_variant() {
 template <int N, int CV = 0> int launch_col_grad(spr_ctx* c, const LossArgs& a, int items) {
     if constexpr (CV < MAX_VARIANTS) {
         if constexpr (same_plan_variant<N, CV>())
-            if (c->colvar == CV) return launch_col_loss_v<N, CV>(c, a, items, false);
+            if (plain_colvar<N>(c) == CV) return launch_col_loss_v<N, CV>(c, a, items, false);
         return launch_col_grad<N, CV + 1>(c, a, items);
     }
     return launch_col_loss_v<N, 0>(c, a, items, false);
@@ -1023,8 +1023,9 @@ template <int N> int launch_col_loss(spr_ctx* c, const LossArgs& a, int items, b
 }
 // The loss pass with one loss partial per workgroup (n / cols_per_wg(n) per
 // field) in the default geometry, and the refinement steps' gradient pass
-// without partials, in the handle's column variant when that variant holds the
-// default radix plan (the same gradients as spr_loss_grad, bit for bit), else in the default geometry too (at 1024^2 the radix-16 variants
+// without partials, in the handle's column variant (the plain projection's) when
+// that variant holds the default radix plan (the same gradients as spr_loss_grad,
+// bit for bit), else in the default geometry too (at 1024^2 the radix-16 variants
 // measured no faster for this pass: 0.577 against 0.575 ms per refinement step).
 int col_loss(spr_ctx* c, const LossArgs& a, int items) { SPR_DISPATCH_N(c, launch_col_loss, c, a, items, true); }
 int col_loss_step(spr_ctx* c, const LossArgs& a, int items) { SPR_DISPATCH_N(c, launch_col_loss, c, a, items, false); }

@@ -205,10 +205,18 @@ SPR_ROW_VARIANT(2048, 5, Plan<2048, 16, 16, 8, 16>, 0, 256, -1, 1, 0, 4, 0, 0, 1
 #undef SPR_COL_VARIANT
 #undef SPR_ROW_VARIANT
 
-// The column variant of the plain projection (k_col) where CV is the compiled choice
-// of the step pass: the same plan in the layout that pass runs best in. 512^2 x 64:
-// 52 us in the skewed tile, 60 in the padded one.
-template <int N, int CV> constexpr int plain_variant() { return N == 512 && CV == 1 ? 6 : CV; }
+// The column variant of the plain projection (k_col) and of the refinement's gradient
+// pass where CV is the compiled choice of the step pass: the same plan in the layout
+// that k_col runs best in, where that differs by more than its 5 % of noise. us per
+// launch, CV / here: 512^2 x 64 62.8 / 50.8, 768^2 x 28 84.0 / 69.9; 256^2 x 128
+// 25.8 in variant 2, 26.0 in variant 1; 384^2 x 64 37.8, the others from 38.8;
+// 1024^2 x 16 67.7 in variant 6, 67.9 in variant 4; 2048^2 x 4 99.5, the others from
+// 100.9.
+template <int N, int CV> constexpr int plain_variant() {
+    if constexpr (N == 512 && CV == 1) return 6;
+    else if constexpr (N == 768 && CV == 2) return 7;
+    else return CV;
+}
 
 constexpr int MAX_VARIANTS = 8;
 template <int N> constexpr int col_variants() {
