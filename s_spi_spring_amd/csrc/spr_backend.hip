@@ -288,7 +288,7 @@ template <int N, int CV> int launch_step_v(spr_ctx* c, const Step& st, int cnt, 
         // Half-width strips while each of them finds a CU of its own.
         const int narrow = narrow_strips<N, G>() && (size_t)cnt * (N / G::C) <= 128 ? 1 : 0;
         const StepArgs a{st.f, st.proj, c->amp, c->amp_of ? c->amp_of + first : nullptr, c->twtab[CV],
-                         c->colmask + (size_t)first * G::T, st.lin_w, st.lin_p, st.all_rows, narrow};
+                         c->colmask + (size_t)first * G::T, c->rowcnt + first, st.lin_w, st.lin_p, st.all_rows, narrow};
         const dim3 grid((unsigned)((size_t)cnt * (N / G::C) << narrow)), block(G::COL_THREADS >> narrow);
         switch (st.mode) {
             case STEP_LIN: hipLaunchKernelGGL((k_col_step<N, STEP_LIN, CV>), grid, block, 0, s, a); break;

@@ -191,7 +191,7 @@ SPR_ROW_VARIANT(1024, 5, RadixPlan<1024>, 0, 256, -1, 1, 0, 4)
 SPR_ROW_VARIANT(2048, 3, RadixPlan<2048>, 0, 256, -1, 1, 0, 4)
 // (plan, -, threads, prefetch, -, -, padding period, -, -, recomputed state): the
 // row update passes recompute rho_n from its row transform instead of reading
-// and writing it, and run on the rows that meet the support (k_row_listed); the
+// and writing it, and run on the listed rows (k_row_listed); the
 // column passes write their projection to a second field buffer (k_col_step)
 SPR_ROW_VARIANT(256, 3, RadixPlan<256>, 0, 256, -1, 1, 0, 4, 0, 0, 1)
 SPR_ROW_VARIANT(384, 3, RadixPlan<384>, 0, 256, -1, 1, 0, 5, 0, 0, 1)
@@ -423,7 +423,15 @@ __device__ __forceinline__ uint8_t support_bit(const uint32_t* __restrict__ bits
 //                      thread of the column pass, thread t of a column)
 // A field whose support is empty lists every row: its rows then run the general
 // update, which keeps the signs of zero that the projection of a vanishing
-// spectrum depends on.
+// spectrum depends on. So does a field of which more than listed_max rows meet the
+// support: the column pass is then the plain projection, which is faster without the
+// others' update and the registers it takes. us per RAAR / HIO iteration with that
+// share of the rows meeting the support, every row listed / only those: 512^2 x 64
+// at 0.92 126/129 against 129/132, at 0.86 126/129 against 125/128; 1024^2 x 16 at
+// 0.92 149/162 against 156/164, at 0.86 149/162 against 150/156; 768^2 x 28, whose
+// strips have four columns, at 0.86 162/169 against 164/173, at 0.80 162/169 against
+// 160/168, at 0.74 162/169 against 152/163.
+constexpr int listed_max(int n) { return n == 768 ? n - n / 5 : n - n / 8; }
 struct SupportPlan {
     const uint8_t* supp;   // 16-byte aligned
     uint32_t* bits;
@@ -481,9 +489,11 @@ __global__ __launch_bounds__(256) void k_row_plan(SupportPlan a) {
             const int u = __shfl_up(sum, o, 64);
             if (tid >= o) sum += u;
         }
-        fw[tid] = f;
-        fbase[tid] = sum - cnt;
-        if (tid == 63) a.rowcnt[p] = sum;
+        const int listed = __shfl(sum, 63, 64);
+        const bool every = listed > listed_max(n);
+        fw[tid] = every ? 0xffffffffu : f;
+        fbase[tid] = every ? 32 * tid : sum - cnt;
+        if (tid == 0) a.rowcnt[p] = every ? n : listed;
     }
     __syncthreads();
     for (int y = tid; y < n; y += 256) {
@@ -513,7 +523,7 @@ __global__ __launch_bounds__((RowVariant<N, RV>::G::ROW_THREADS)) void k_row(Row
     constexpr int V = G::V, T = G::T;
     constexpr int PREFETCH = G::ROW_PREFETCH >= 0 ? G::ROW_PREFETCH : SPR_ROW_PREFETCH;
     constexpr bool WV = T <= 64;   // every row inside one wavefront: no workgroup barriers
-        __shared__ float2 tw[TwTableP<PL>::SIZE];
+    __shared__ float2 tw[TwTableP<PL>::SIZE];
     __shared__ float2 lds[G::RW * G::RS];
     const int tid = threadIdx.x;
     const int t = tid % T;
@@ -589,10 +599,12 @@ __global__ __launch_bounds__((RowVariant<N, RV>::G::ROW_THREADS)) void k_row(Row
 
 // Row update of an iteration that recomputes rho_n: the rows that meet the
 // support, RW at a time (the column pass, k_col_step, has updated the others).
-// Workgroup b takes field b % fields and group b / fields of its list; those past
-// the lists' ends come last and leave at once (4096 workgroups that step through
-// the lists instead took the same time: 20 us at 512^2 x 64 with 22 % of the rows
-// listed, against 60 us for the pass over every row).
+// The workgroups take the first groups of every field's list, then the next ones, so
+// that those past the lists' ends come last and leave at once (4096 workgroups that
+// step through the lists instead took the same time: 20 us at 512^2 x 64 with 22 %
+// of the rows listed, against 60 us for the pass over every row). With two rows in a
+// workgroup eight workgroups in a row stay in one field: 1024^2 x 16 with every row
+// listed 149/162 us per RAAR/HIO iteration against 155/166, even with a quarter.
 template <int N, int MODE, int RV>
 __global__ __launch_bounds__((RowVariant<N, RV>::G::ROW_THREADS)) void k_row_listed(RowArgs a, int fields) {
     using G = typename RowVariant<N, RV>::G;
@@ -604,9 +616,12 @@ __global__ __launch_bounds__((RowVariant<N, RV>::G::ROW_THREADS)) void k_row_lis
     const int tid = threadIdx.x;
     const int t = tid % T;
     const int rl = tid / T;
-    const int field = blockIdx.x % fields;
+    constexpr int RUN = RW <= 2 ? 8 : 1;   // workgroups in a row in one field
+    static_assert(N / RW % RUN == 0, "a field's groups fill whole runs");
+    const int run = blockIdx.x / RUN;
+    const int field = run % fields;
     const int listed = a.rowcnt[field];
-    const int first = blockIdx.x / fields * RW;
+    const int first = (run / fields * RUN + (int)(blockIdx.x % RUN)) * RW;
     if (first >= listed) return;
     tw_fill_p<PL>(tw, a.tw, tid, G::ROW_THREADS);
     // Block-uniform bases with 32-bit per-thread offsets (SGPR base addressing).
@@ -616,9 +631,12 @@ __global__ __launch_bounds__((RowVariant<N, RV>::G::ROW_THREADS)) void k_row_lis
     const uint16_t* __restrict__ list = a.rowlist + (size_t)field * N;
     const RowAccT<G::ROW_PAD_SHIFT> acc{lds + rl * G::RS};
     __syncthreads();
-    // Past the list's end a line repeats the last row and stores nothing.
+    // Past the list's end a line repeats the last row and stores nothing. A list of
+    // every row is not read.
     const bool live = first + rl < listed;
-    const int off = list[live ? first + rl : listed - 1] * N + t;
+    int row = live ? first + rl : listed - 1;
+    if (listed != N) row = list[row];
+    const int off = row * N + t;
     float2 v[V];
     // rho' = rowIFFT(proj)/N^2 and rho_n = rowIFFT(work)/N, the state recomputed
     // from its row transform (within float rounding); ER needs rho' only, which
@@ -826,7 +844,8 @@ struct StepArgs {
     const float* amp;   // amplitudes [patterns][N][N]
     const int* amp_of;  // field -> pattern (NULL: pattern 0)
     const float2* twtab;      // the plan's twiddle table
-    const uint32_t* colmask;  // [fields][N/V] row masks of k_pack_support
+    const uint32_t* colmask;  // [fields][N/V] row masks of k_row_plan
+    const int* rowcnt;        // [fields] rows listed by k_row_plan
     float lin_w, lin_p;       // STEP_LIN: f <- lin_w f + lin_p projected outside the support
     int all_rows;             // STEP_ER*: rho_n is any density (the first pass of a block)
     int narrow;               // 1: strips of C/2 columns (narrow_strips), 0: of C
@@ -869,6 +888,36 @@ __device__ __forceinline__ int row_offset(int voff, uint32_t off_rows, int q) {
     return voff | (int)((off_rows << (31 - q)) & 0x80000000u);
 }
 
+// STEP_LIN of a field whose every row is listed: the plain projection, into proj,
+// in the tile layout that is best for it (plain_variant), which the registers of the
+// other path do not leave room for.
+template <int N, class G>
+__device__ __forceinline__ void step_every_row(const StepArgs& a, float2* lds, const float2* tw, int p, int t, int c, int x0) {
+    using PL = typename G::PL;
+    constexpr int V = G::V, T = G::T, C = G::C;
+    constexpr int SKEW = G::COL_SKEW > 0 ? G::COL_SKEW : (N == 512 || N == 768) && G::CS == C + 1 ? log2i(C) : 0;
+    using Acc = std::conditional_t<(SKEW > 0), ColAccSkew<C, (SKEW > 0 ? SKEW : 1)>, ColAcc<G::CS>>;
+    static_assert(SKEW == 0 || (N + (N >> SKEW)) * C <= G::COL_TILE, "the skewed tile fits in the padded one");
+    const float2* __restrict__ f = a.f + (size_t)p * N * N + x0;
+    const float* __restrict__ amp = a.amp + amp_offset<N>(a.amp_of, p) + x0;
+    float2* __restrict__ proj = a.proj + (size_t)p * N * N + x0;
+    const int off = t * N + c;
+    const Acc acc{lds + c};
+    float2 v[V];
+    float am[V];
+#pragma unroll
+    for (int r = 0; r < V; ++r) v[r] = f[off + r * T * N];
+#pragma unroll
+    for (int q = 0; q < V; ++q) am[q] = amp[off + q * T * N];
+    __syncthreads();   // twiddle table
+    fft_line_p<PL, +1>(v, acc, tw, t);
+#pragma unroll
+    for (int q = 0; q < V; ++q) v[q] = project_modulus(v[q], am[q]);
+    fft_line_p<PL, -1>(v, acc, tw, t);
+#pragma unroll
+    for (int q = 0; q < V; ++q) proj[off + q * T * N] = v[q];
+}
+
 // Columns [x0, x0 + C) of one field. Outside the support (s = 0) the update is
 // linear in rho_n and rho', so it can be made on their row transforms, f and
 // proj/N = rowFFT(rho'):
@@ -908,13 +957,19 @@ __attribute__((amdgpu_waves_per_eu((ColVariant<N, CV>::G::COL_WAVES_PER_EU)))) v
     const int strip = col_strip<N>(blockIdx.x, lc);
     const int p = (strip >> narrow) / TILES;
     const int x0 = (strip - p * (TILES << narrow)) << lc;
-    const uint32_t off_rows = ~a.colmask[(size_t)p * T + t];
     const float2* tw = twl;
     if constexpr (G::TW_GLOBAL) {
         tw = a.twtab;
     } else {
         for (int e = tid; e < TwTableP<PL>::SIZE; e += T << lc) twl[e] = a.twtab[e];
     }
+    if constexpr (MODE == STEP_LIN) {
+        if (a.rowcnt[p] == N) {
+            step_every_row<N, G>(a, lds, tw, p, t, c, x0);
+            return;
+        }
+    }
+    const uint32_t off_rows = ~a.colmask[(size_t)p * T + t];
     const __amdgpu_buffer_rsrc_t bf = field_buffer<N, 8>(a.f + (size_t)p * N * N);
     const __amdgpu_buffer_rsrc_t ba = field_buffer<N, 4>(a.amp + amp_offset<N>(a.amp_of, p));
     const int off = t * N + x0 + c;
