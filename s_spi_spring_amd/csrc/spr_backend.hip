@@ -714,16 +714,20 @@ int col_lines(int n, int cv) {
     return 0;
 }
 
-// The support bits, row lists and column masks of all resident individuals, for
-// the handle's current column variant.
+// Where the supports' forms of individuals from `first` on lie; the row lists and
+// column masks, for the handle's current column variant, only where rho_n is recomputed.
+SupportPlan support_plan(const spr_ctx* c, int first) {
+    const size_t f = (size_t)first, np = (size_t)c->n * c->n;
+    const int lines = row_recomputes(c->n, c->rowvar) ? col_lines(c->n, c->colvar) : 0;
+    return SupportPlan{c->supp + f * np,        c->sbits + f * (np / 32), c->rowcnt + f, c->rowlist + f * c->n,
+                       c->colmask + f * lines, c->rowflags + f * (c->n / 32), c->n, lines};
+}
+// The support bits of all resident individuals, and the flags that the first row pass
+// makes row lists and column masks from.
 int pack_support(spr_ctx* c, hipStream_t s) {
     if (c->P <= 0) return SPR_OK;
-    const SupportPlan a{c->supp, c->sbits, c->rowcnt, c->rowlist, c->colmask, c->rowflags, c->n,
-                        col_lines(c->n, c->colvar)};
-    hipLaunchKernelGGL(k_pack_support, dim3((unsigned)(c->n / 32 * c->P)), dim3(256), 0, s, a);
-    SPR_HIP(c, hipGetLastError());
-    if (!row_recomputes(c->n, c->rowvar)) return SPR_OK;
-    hipLaunchKernelGGL(k_row_plan, dim3((unsigned)c->P), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(k_pack_support, dim3((unsigned)(c->n / 32 * c->P)), dim3(pack_threads(c->n)), 0, s,
+                       support_plan(c, 0));
     SPR_HIP(c, hipGetLastError());
     return SPR_OK;
 }
@@ -731,7 +735,7 @@ int pack_support(spr_ctx* c, hipStream_t s) {
 // The projection pass of iteration i of a block (i = niter: the trailing one) over
 // individuals [first, first + cnt), whose fields `a` points to.
 int project(spr_ctx* c, int row_mode, const RowArgs& a, bool rs, int i, int niter, int cnt, hipStream_t s, int first) {
-    if (!rs || (i == niter && row_mode != ROW_ER)) return col_n(c, COL_PROJ, a.work, cnt, s, first);
+    if (!rs || (i == niter && (row_mode != ROW_ER || niter == 0))) return col_n(c, COL_PROJ, a.work, cnt, s, first);
     Step st{STEP_LIN, a.work, const_cast<float2*>(a.proj), 1.f, -(a.beta * a.inv_n), 0};
     if (row_mode == ROW_RAAR) {
         st.lin_w = a.beta;
@@ -753,8 +757,13 @@ int queue_iterate_lanes(spr_ctx* c, int mode, int niter, const RowArgs& a0) {
     const int h = (c->P + 1) / 2, h2 = c->P - h;
     const size_t off = (size_t)h * c->n * c->n;
     const bool rs = row_recomputes(c->n, c->rowvar);
-    const RowArgs a = a0;
+    RowArgs a = a0;
+    if (niter > 0) {
+        SPR_TRY(pack_support(c, c->stream));
+        a.plan = support_plan(c, 0);
+    }
     RowArgs b = a;
+    if (niter > 0) b.plan = support_plan(c, h);
     b.rho += off;
     b.work += off;
     b.supp += off;
@@ -763,7 +772,6 @@ int queue_iterate_lanes(spr_ctx* c, int mode, int niter, const RowArgs& a0) {
     b.rowlist += (size_t)h * c->n;
     b.proj += off;
     hipStream_t s1 = c->stream, s2 = c->lane2;
-    SPR_TRY(pack_support(c, s1));
     SPR_TRY(row_n(c, ROW_FWD, a, h, s1));
     SPR_HIP(c, hipEventRecord(c->ev_fork, s1));
     SPR_HIP(c, hipStreamWaitEvent(s2, c->ev_fork, 0));
@@ -804,10 +812,11 @@ int queue_iterate_block(spr_ctx* c, int mode, int niter, const RowArgs& a0) {
     const int chunk = chunk_individuals(c);
     const size_t np = (size_t)c->n * c->n;
     const bool rs = row_recomputes(c->n, c->rowvar);
-    SPR_TRY(pack_support(c, c->stream));
+    if (niter > 0) SPR_TRY(pack_support(c, c->stream));
     for (int first = 0; first < c->P; first += chunk) {
         const int cnt = std::min(chunk, c->P - first);
         RowArgs a = a0;
+        if (niter > 0) a.plan = support_plan(c, first);
         a.rho += first * np;
         a.work += first * np;
         a.supp += first * np;
@@ -1200,7 +1209,8 @@ VariantPair default_variants(int n) {
 int time_iteration(spr_ctx* c, const RowArgs& ra0, int reps, hipEvent_t e0, hipEvent_t e1, float* ms) {
     RowArgs ra = ra0;
     const bool rs = row_recomputes(c->n, c->rowvar);
-    SPR_TRY(pack_support(c, c->stream));   // the column masks follow the column variant
+    SPR_TRY(pack_support(c, c->stream));
+    ra.plan = support_plan(c, 0);   // the column masks follow the column variant
     SPR_TRY(row_n(c, ROW_FWD, ra, c->P, c->stream));
     if (!rs) {
         const int np = c->n * c->n;

@@ -392,29 +392,6 @@ enum RowMode {
     ROW_INV_INPLACE = 6,   // rho <- rowFFT-(rho)/N^2 (2-D IFT, second half)
 };
 
-struct RowArgs {
-    float2* rho;
-    float2* work;
-    const uint8_t* supp;     // supports, one byte per pixel (on-chip blocks)
-    const uint32_t* sbits;   // supports, one bit per pixel (row update passes)
-    const float2* tw;
-    float beta;
-    float inv_nn;  // 1/N^2 (exact for power-of-two N; within 1 ulp of dividing by N^2 otherwise)
-    PhaseCut pc;
-    const float2* proj;  // column-projected fields, read by variants that recompute rho_n
-    float inv_n;         // 1/N
-    // Rows that meet the support (variants that recompute rho_n): per field
-    // their number and, ascending, their indices.
-    const int* rowcnt;       // [fields]
-    const uint16_t* rowlist; // [fields][N]
-};
-
-// Support bit of pixel i of a field: bit i&31 of word i>>5 (N*N and the
-// row-block offsets are multiples of 32).
-__device__ __forceinline__ uint8_t support_bit(const uint32_t* __restrict__ bits, int i) {
-    return (uint8_t)((bits[i >> 5] >> (i & 31)) & 1u);
-}
-
 // The supports of a block in the forms its passes read, per field:
 //   bits     [N*N/32]  word w holds pixels [32w, 32w+32), bit k = (supp[32w+k] != 0)
 //   rowcnt             number of rows that meet the support
@@ -438,16 +415,42 @@ struct SupportPlan {
     int* rowcnt;
     uint16_t* rowlist;
     uint32_t* colmask;
-    uint32_t* rowflags;    // [N/32] one bit per row, from k_pack_support to k_row_plan
+    uint32_t* rowflags;    // [N/32] one bit per row, from k_pack_support to row_plan
     int n;
     int lines;             // entries of colmask per field: N/V
 };
 
-// N/32 workgroups per field, 32 rows each: a thread packs 32 bytes at a time, as
-// two 16-byte loads. (One workgroup per field doing both kernels' work took 40 us
-// at 1024^2 x 32 and 14 us at 512^2 x 64; workgroups handing their flags to the
-// last one of the field 45 and 32 us, in agent-scope fences.)
-__global__ __launch_bounds__(256) void k_pack_support(SupportPlan a) {
+struct RowArgs {
+    float2* rho;
+    float2* work;
+    const uint8_t* supp;     // supports, one byte per pixel (on-chip blocks)
+    const uint32_t* sbits;   // supports, one bit per pixel (row update passes)
+    const float2* tw;
+    float beta;
+    float inv_nn;  // 1/N^2 (exact for power-of-two N; within 1 ulp of dividing by N^2 otherwise)
+    PhaseCut pc;
+    const float2* proj;  // column-projected fields, read by variants that recompute rho_n
+    float inv_n;         // 1/N
+    // Rows that meet the support (variants that recompute rho_n): per field
+    // their number and, ascending, their indices.
+    const int* rowcnt;       // [fields]
+    const uint16_t* rowlist; // [fields][N]
+    SupportPlan plan;        // ROW_FWD: made for each field where plan.lines > 0
+};
+
+// Support bit of pixel i of a field: bit i&31 of word i>>5 (N*N and the
+// row-block offsets are multiples of 32).
+__device__ __forceinline__ uint8_t support_bit(const uint32_t* __restrict__ bits, int i) {
+    return (uint8_t)((bits[i >> 5] >> (i & 31)) & 1u);
+}
+
+// N/32 workgroups per field, 32 rows each: a thread packs 32 bytes, as two 16-byte
+// loads. The lists follow from all flags of a field, in the first row pass
+// (row_plan). (One workgroup per field packing and listing took 40 us at 1024^2 x 32
+// and 14 us at 512^2 x 64; workgroups handing their flags to the last one of the
+// field 45 and 32 us, in agent-scope fences.)
+constexpr int pack_threads(int n) { return n < 1024 ? n : 1024; }
+__global__ __launch_bounds__(1024) void k_pack_support(SupportPlan a) {
     __shared__ uint32_t hit;
     const int tid = threadIdx.x, n = a.n, wpr = n / 32;
     const size_t blk = blockIdx.x;   // field * wpr + 32-row group
@@ -456,7 +459,7 @@ __global__ __launch_bounds__(256) void k_pack_support(SupportPlan a) {
     if (tid == 0) hit = 0;
     __syncthreads();
     uint32_t rows = 0;
-    for (int w = tid; w < n; w += 256) {
+    for (int w = tid; w < n; w += pack_threads(n)) {
         const uint4 lo = *reinterpret_cast<const uint4*>(supp + 32 * w);
         const uint4 hi = *reinterpret_cast<const uint4*>(supp + 32 * w + 16);
         const unsigned x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
@@ -473,12 +476,16 @@ __global__ __launch_bounds__(256) void k_pack_support(SupportPlan a) {
     if (tid == 0) a.rowflags[blk] = hit;
 }
 
-// Row list and column masks of one field per workgroup.
-__global__ __launch_bounds__(256) void k_row_plan(SupportPlan a) {
-    __shared__ uint32_t fw[64];   // one bit per row (N <= 2048)
-    __shared__ int fbase[64];     // rows listed before each word
-    const int tid = threadIdx.x, n = a.n, wpr = n / 32;
-    const size_t p = blockIdx.x;
+// Row list and column masks of field p, by one workgroup of NT >= 64 threads; 512 bytes
+// of LDS at `lds`. The workgroup of a field's first rows does this in the first row
+// pass of a block: as a kernel of its own it held up every block by 3 - 5 us, and in
+// workgroups of its own in that pass by 1 - 3 (1024^2 x 1, one RAAR iteration: 68.7,
+// 69.9 and here 66.7 us).
+template <int N, int NT> __device__ __forceinline__ void row_plan(const SupportPlan& a, size_t p, void* lds) {
+    uint32_t* const fw = static_cast<uint32_t*>(lds);       // one bit per row (N <= 2048)
+    int* const fbase = static_cast<int*>(lds) + 64;         // rows listed before each word
+    constexpr int n = N, wpr = N / 32;
+    const int tid = threadIdx.x;
     if (tid < 64) {   // running sum of the flag words in one wavefront
         uint32_t f = tid < wpr ? a.rowflags[p * wpr + tid] : 0u;
         if (__ballot(f != 0u) == 0) f = tid < wpr ? 0xffffffffu : 0u;
@@ -496,12 +503,12 @@ __global__ __launch_bounds__(256) void k_row_plan(SupportPlan a) {
         if (tid == 0) a.rowcnt[p] = every ? n : listed;
     }
     __syncthreads();
-    for (int y = tid; y < n; y += 256) {
+    for (int y = tid; y < n; y += NT) {
         const uint32_t f = fw[y >> 5];
         if ((f >> (y & 31)) & 1u)
             a.rowlist[p * n + fbase[y >> 5] + __popc(f & ((1u << (y & 31)) - 1u))] = (uint16_t)y;
     }
-    for (int t = tid; t < a.lines; t += 256) {
+    for (int t = tid; t < a.lines; t += NT) {
         uint32_t m = 0;
         for (int y = t, q = 0; y < n; y += a.lines, ++q) m |= ((fw[y >> 5] >> (y & 31)) & 1u) << q;
         a.colmask[p * a.lines + t] = m;
@@ -546,6 +553,13 @@ __global__ __launch_bounds__((RowVariant<N, RV>::G::ROW_THREADS)) void k_row(Row
         float2* dst = (MODE == ROW_FWD) ? work : rho;
 #pragma unroll
         for (int q = 0; q < V; ++q) dst[off + q * T] = v[q];
+        if constexpr (MODE == ROW_FWD && G::ROW_RECOMPUTE) {
+            constexpr int GROUPS = N / G::RW;   // workgroups per field
+            if (a.plan.lines > 0 && blockIdx.x % GROUPS == 0) {
+                __syncthreads();
+                row_plan<N, G::ROW_THREADS>(a.plan, blockIdx.x / GROUPS, lds);
+            }
+        }
     } else if constexpr (MODE == ROW_FINAL || MODE == ROW_INV_INPLACE) {
         const float2* src = (MODE == ROW_FINAL) ? work : rho;
 #pragma unroll
@@ -844,8 +858,8 @@ struct StepArgs {
     const float* amp;   // amplitudes [patterns][N][N]
     const int* amp_of;  // field -> pattern (NULL: pattern 0)
     const float2* twtab;      // the plan's twiddle table
-    const uint32_t* colmask;  // [fields][N/V] row masks of k_row_plan
-    const int* rowcnt;        // [fields] rows listed by k_row_plan
+    const uint32_t* colmask;  // [fields][N/V] row masks of row_plan
+    const int* rowcnt;        // [fields] rows listed by row_plan
     float lin_w, lin_p;       // STEP_LIN: f <- lin_w f + lin_p projected outside the support
     int all_rows;             // STEP_ER*: rho_n is any density (the first pass of a block)
     int narrow;               // 1: strips of C/2 columns (narrow_strips), 0: of C
