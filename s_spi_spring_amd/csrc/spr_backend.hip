@@ -56,7 +56,7 @@ struct spr_ctx {
     float2* work2 = nullptr;      // second half-transformed field per individual (correlations, |b|)
     uint8_t* supp = nullptr;
     uint32_t* sbits = nullptr;    // supports one bit per pixel, packed at the start of every iteration block
-    void* planbuf = nullptr;      // the allocation of corrwin and the next four
+                                  // (its allocation also holds corrwin and the next four)
     // Rows that meet each support, made with sbits (SupportPlan in spr_kernels.hpp).
     int* rowcnt = nullptr;        // [cap]
     uint16_t* rowlist = nullptr;  // [cap][n]
@@ -68,8 +68,7 @@ struct spr_ctx {
     int npat = 1;                 // patterns sharing this handle (one amplitude each)
     int colvar = 0, rowvar = 0;   // variants of the column and row iteration passes
     bool exact = false;           // chosen by the caller or the autotuner: the plain projection runs colvar itself
-    float2* twbuf = nullptr;           // twiddle tables of the column variants
-    float2* twtab[MAX_VARIANTS] = {};  // each variant's, in twbuf
+    const float2* twtab[MAX_VARIANTS] = {};  // twiddle tables of the column variants, behind tw
     size_t chunk_bytes = 0;       // iteration blocks run in chunks of this working set (0: whole population)
     int fused = -1;               // on-chip iteration blocks (N <= 128): -1 by population size, 0 never, 1 always
     int* amp_of = nullptr;        // slot -> pattern when npat > 1, else NULL
@@ -313,31 +312,42 @@ template <int N, int CV = 0> int launch_step(spr_ctx* c, const Step& st, int cnt
     }
 }
 
-// Twiddle tables of every column variant of size N (read by the step passes, and
-// by the column passes of variants with TW_GLOBAL), one after another in one
-// allocation.
-template <int N, int CV = 0> constexpr size_t twtab_entries() {
-    if constexpr (CV < MAX_VARIANTS) {
-        size_t n = 0;
-        if constexpr (ColVariant<N, CV>::valid) n = TwTableP<typename ColVariant<N, CV>::G::PL>::SIZE;
-        return n + twtab_entries<N, CV + 1>();
+// Stage S and on of plan PL's twiddle table (TwTableP), from the roots exp(-2 pi i m/N).
+template <class PL, int S = 1> void append_twtab(const std::vector<float2>& root, std::vector<float2>& out) {
+    if constexpr (S < PL::ns) {
+        constexpr int R = PL::r[S], NS = span_before<PL>(S);
+        for (int k = 0; k < NS; ++k)
+            for (int r = 1; r < R; ++r) out.push_back(root[r * k * (PL::N / (NS * R))]);
+        append_twtab<PL, S + 1>(root, out);
     }
-    return 0;
 }
-template <int N, int CV = 0> int build_twtabs(spr_ctx* c, size_t at = 0) {
-    if constexpr (CV < MAX_VARIANTS) {
-        if constexpr (CV == 0) SPR_HIP(c, hipMalloc(&c->twbuf, twtab_entries<N>() * sizeof(float2)));
-        if constexpr (ColVariant<N, CV>::valid) {
-            using G = typename ColVariant<N, CV>::G;
-            c->twtab[CV] = c->twbuf + at;
-            at += TwTableP<typename G::PL>::SIZE;
-            hipLaunchKernelGGL((k_build_twtab<typename G::PL>), dim3(1), dim3(256), 0, c->stream, c->twtab[CV],
-                               (const float2*)c->tw);
-            SPR_HIP(c, hipGetLastError());
-        }
-        return build_twtabs<N, CV + 1>(c, at);
+// The first column variant of size N with the plan of variant CV.
+template <int N, int CV, int FIRST = 0> constexpr int first_of_plan() {
+    if constexpr (FIRST < CV) {
+        if constexpr (ColVariant<N, FIRST>::valid)
+            if (std::is_same<typename ColVariant<N, FIRST>::G::PL::Table, typename ColVariant<N, CV>::G::PL::Table>::value)
+                return FIRST;
+        return first_of_plan<N, CV, FIRST + 1>();
     }
-    return SPR_OK;
+    return CV;
+}
+// Twiddle tables of the column variants of size N, one per radix plan, behind the roots
+// in `t`: read by the step passes, and by the column passes of variants with
+// TW_GLOBAL. at[CV] is where variant CV's begins (0: no pass reads it).
+template <int N, int CV = 0> void append_twtabs(const std::vector<float2>& root, std::vector<float2>& t, size_t* at) {
+    if constexpr (CV < MAX_VARIANTS) {
+        if constexpr (ColVariant<N, CV>::valid) {
+            if constexpr (has_recompute<N>() || ColVariant<N, CV>::G::TW_GLOBAL) {
+                constexpr int F = first_of_plan<N, CV>();
+                if (at[F] == 0) {
+                    at[F] = t.size();
+                    append_twtab<typename ColVariant<N, CV>::G::PL>(root, t);
+                }
+                at[CV] = at[F];
+            }
+        }
+        append_twtabs<N, CV + 1>(root, t, at);
+    }
 }
 
 // Column variant of the plain projection: the handle's, or, where the handle runs
@@ -1463,12 +1473,11 @@ static int create_context(spr_ctx** out, int n, int capacity, int npat, const fl
     if ((e = hipMalloc(&c->work, np * capacity * sizeof(float2))) != hipSuccess)
         return cleanup_fail("hipMalloc work", e);
     if ((e = hipMalloc(&c->supp, np * capacity)) != hipSuccess) return cleanup_fail("hipMalloc supp", e);
-    if ((e = hipMalloc(&c->sbits, np / 8 * capacity)) != hipSuccess) return cleanup_fail("hipMalloc sbits", e);
     {   // 4-byte arrays first, the 2-byte row lists last
-        const size_t cap = (size_t)capacity, masks = cap * (n / 8), flags = cap * (n / 32);
-        if ((e = hipMalloc(&c->planbuf, (np + masks + flags + cap) * 4 + cap * n * sizeof(uint16_t))) != hipSuccess)
-            return cleanup_fail("hipMalloc row lists", e);
-        c->corrwin = (float*)c->planbuf;
+        const size_t cap = (size_t)capacity, bits = np / 32 * cap, masks = cap * (n / 8), flags = cap * (n / 32);
+        if ((e = hipMalloc(&c->sbits, (bits + np + masks + flags + cap) * 4 + cap * n * sizeof(uint16_t))) != hipSuccess)
+            return cleanup_fail("hipMalloc sbits", e);
+        c->corrwin = (float*)(c->sbits + bits);
         c->colmask = (uint32_t*)(c->corrwin + np);
         c->rowflags = c->colmask + masks;
         c->rowcnt = (int*)(c->rowflags + flags);
@@ -1476,7 +1485,6 @@ static int create_context(spr_ctx** out, int n, int capacity, int npat, const fl
     }
     if ((e = hipMalloc(&c->amp, np * npat * sizeof(float))) != hipSuccess) return cleanup_fail("hipMalloc amp", e);
     if ((e = hipMalloc(&c->amp_t, np * npat * sizeof(float))) != hipSuccess) return cleanup_fail("hipMalloc amp_t", e);
-    if ((e = hipMalloc(&c->tw, n * sizeof(float2))) != hipSuccess) return cleanup_fail("hipMalloc tw", e);
     if ((e = hipMalloc(&c->work2, np * capacity * sizeof(float2))) != hipSuccess)
         return cleanup_fail("hipMalloc work2", e);
     {
@@ -1501,27 +1509,20 @@ static int create_context(spr_ctx** out, int n, int capacity, int npat, const fl
         if ((e = hipMemcpy(c->amp_of, amp_of, (size_t)capacity * sizeof(int), hipMemcpyHostToDevice)) != hipSuccess)
             return cleanup_fail("upload pattern map", e);
     }
-    std::vector<float2> tw(n);
+    std::vector<float2> root(n);
     for (int k = 0; k < n; ++k) {
         const double ang = -2.0 * M_PI * (double)k / (double)n;
-        tw[k] = make_float2((float)std::cos(ang), (float)std::sin(ang));
+        root[k] = make_float2((float)std::cos(ang), (float)std::sin(ang));
     }
-    if ((e = hipMemcpy(c->tw, tw.data(), n * sizeof(float2), hipMemcpyHostToDevice)) != hipSuccess)
+    std::vector<float2> tw = root;
+    size_t tab[MAX_VARIANTS] = {};
+#define SPR_TW_CASE(N_) if (n == N_) append_twtabs<N_>(root, tw, tab);
+    SPR_SIZES(SPR_TW_CASE)
+#undef SPR_TW_CASE
+    if ((e = hipMalloc(&c->tw, tw.size() * sizeof(float2))) != hipSuccess) return cleanup_fail("hipMalloc tw", e);
+    for (int v = 0; v < MAX_VARIANTS; ++v) c->twtab[v] = tab[v] ? c->tw + tab[v] : nullptr;
+    if ((e = hipMemcpy(c->tw, tw.data(), tw.size() * sizeof(float2), hipMemcpyHostToDevice)) != hipSuccess)
         return cleanup_fail("upload twiddles", e);
-    {
-        int rc = SPR_ERR_ARG;
-        switch (n) {
-#define SPR_TWTAB_CASE(N_) \
-    case N_: rc = build_twtabs<N_>(c); break;
-            SPR_SIZES(SPR_TWTAB_CASE)
-#undef SPR_TWTAB_CASE
-        }
-        if (rc != SPR_OK || (e = hipStreamSynchronize(c->stream)) != hipSuccess) {
-            g_create_error = "twiddle tables: " + c->err;
-            spr_destroy(c);
-            return SPR_ERR_HIP;
-        }
-    }
     for (int k = 0; k < npat; ++k) {
         if ((e = hipMemcpy(c->amp + k * np, amps[k], np * sizeof(float), hipMemcpyHostToDevice)) != hipSuccess)
             return cleanup_fail("upload amplitude", e);
@@ -1550,9 +1551,7 @@ int spr_destroy(spr_ctx* c) {
     (void)hipFree(c->sbits);
     (void)hipFree(c->amp);
     (void)hipFree(c->amp_t);
-    (void)hipFree(c->planbuf);
     (void)hipFree(c->amp_of);
-    (void)hipFree(c->twbuf);
     (void)hipFree(c->tw);
     (void)hipFree(c->work2);
     (void)hipFree(c->partial);

@@ -209,6 +209,7 @@ template <int R, int S> __device__ __forceinline__ void dftR(float2* v) {
 // A radix plan: the N-point transform with V values per thread in ns stages of
 // radices r[] (each dividing V; unused entries 0).
 template <int N_, int V_, int R0, int R1, int R2 = 0, int R3 = 0> struct Plan {
+    using Table = Plan;   // plans of one Table share their twiddle table
     static constexpr int N = N_;
     static constexpr int V = V_;
     static constexpr int ns = R2 == 0 ? 2 : R3 == 0 ? 3 : 4;

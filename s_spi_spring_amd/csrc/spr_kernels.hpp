@@ -1034,10 +1034,4 @@ __attribute__((amdgpu_waves_per_eu((ColVariant<N, CV>::G::COL_WAVES_PER_EU)))) v
 
 namespace spr {
 
-// The twiddle table of plan PL in global memory (one workgroup), for the
-// column-pass variants that read it from there.
-template <class PL> __global__ void k_build_twtab(float2* out, const float2* __restrict__ root) {
-    tw_fill_p<PL>(out, root, threadIdx.x, blockDim.x);
-}
-
 }  // namespace spr
