@@ -156,6 +156,7 @@ SPR_COL_VARIANT(1024, 1, Plan<1024, 16, 16, 8, 8>, 8, 256, -1, 1, 1, 3, 0, 4)
 SPR_COL_VARIANT(1024, 3, Plan<1024, 16, 16, 8, 8>, 8, 256, -1, 0, 1, 3, 0, 4)
 SPR_COL_VARIANT(1024, 5, Plan<1024, 16, 16, 8, 8>, 8, 256, -1, 1, 1)
 SPR_COL_VARIANT(1024, 6, Plan<1024, 16, 16, 8, 8>, 8, 256, -1, 0, 0)
+SPR_COL_VARIANT(1024, 7, RadixPlan<1024>, 8, 256, -1, 1, 1)
 SPR_COL_VARIANT(2048, 1, RadixPlan<2048>, 4, 256, -1, 0, 1)
 SPR_COL_VARIANT(2048, 2, Plan<2048, 16, 16, 8, 16>, 8, 256, -1, 0, 1)
 // (plan, columns, -, -, -, -, -, spare tile row every 2^k rows, waves per SIMD):
@@ -167,7 +168,6 @@ SPR_COL_VARIANT(512, 6, RadixPlan<512>, 8, 256, -1, 0, 0, 3, 3)
 SPR_COL_VARIANT(512, 7, RadixPlan<512>, 4, 256, -1, 0, 0, 3, 2, 5)
 SPR_COL_VARIANT(768, 1, RadixPlan<768>, 4, 256, -1, 1, 0, 3, 2, 3)
 SPR_COL_VARIANT(768, 6, RadixPlan<768>, 4, 256, -1, 0, 0, 3, 2)
-SPR_COL_VARIANT(1024, 7, Plan<1024, 16, 16, 8, 8>, 4, 256, -1, 0, 0, 3, 4, 3)
 // row variants: plan, -, threads per workgroup, prefetch mode
 SPR_ROW_VARIANT(256, 1, RadixPlan<256>, 0, 512)
 SPR_ROW_VARIANT(384, 1, RadixPlan<384>, 0, 512)
