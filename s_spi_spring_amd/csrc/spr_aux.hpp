@@ -81,9 +81,11 @@ __device__ __forceinline__ unsigned long long block_max_u64(unsigned long long v
 }
 
 // Column passes outside the iteration: tiles of 8 columns where the default is
-// wider, 16 up to 128^2 (whole 128-byte lines). A workgroup then has 4 - 8
-// wavefronts instead of 16, so that the correlation passes, which hold two fields'
-// values (94 registers), keep 3 - 4 workgroups on a CU instead of one.
+// wider, 16 up to 128^2 (whole 128-byte lines). A workgroup then has 4 wavefronts at
+// 256^2 and 384^2 (16 and 8 in the default tile) and 8 at 512^2 (16), so that the
+// correlation passes, which hold two fields' values (72 - 79 registers, 117 with 12
+// values per thread), keep 6, 4 and 3 workgroups on a CU. From 768^2 on the default is
+// no wider: two workgroups of 8 wavefronts at 768^2, one of 16 above.
 template <int N> constexpr int aux_columns() { return N <= 128 ? 16 : Geo<N>::C < 8 ? Geo<N>::C : 8; }
 template <int N> using AuxGeo = GeoT<N, RadixPlan<N>, aux_columns<N>()>;
 
@@ -299,10 +301,8 @@ struct AuxColArgs {
     float sigma_ft;
     double* partial;
     unsigned* maxbits;
-    const float2* ref;          // ACOL_CORR reference spectra (base of a batch)
-    const int* ref_index;       // item -> reference spectrum (NULL: the item's own transformed field)
+    const float2* ref;          // ACOL_CORR reference spectrum (NULL: each item's own)
     const float* win;           // ACOL_CORR: k_corr_window's table
-    int unit_scale;             // ACOL_CORR: apply normalize_ft_shift to d first
 };
 
 // normalize_ft_shift with e = 1: z |z|/|z|.
@@ -388,11 +388,11 @@ __global__ __launch_bounds__(AuxGeo<N>::COL_THREADS) void k_col_aux(AuxColArgs a
         // and only the second product waits in registers:
         // sign -1: (conj d) r ; sign +1: d r ; both weighted and masked.
         float2 v2[V];
-        const float2* __restrict__ ref = a.ref ? a.ref + (size_t)(a.ref_index ? a.ref_index[item] : 0) * N * N + x0 + c : nullptr;
+        const float2* __restrict__ ref = a.ref ? a.ref + x0 + c : nullptr;
 #pragma unroll
         for (int q = 0; q < V; ++q) {
             const int ky = t + q * T;
-            const float2 d = a.unit_scale ? unit_scaled(v[q]) : v[q];
+            const float2 d = unit_scaled(v[q]);   // normalize_ft_shift, as in the reference's spectrum
             const float2 r = ref ? ref[(size_t)ky * N] : d;   // symmetry: the spectrum with itself
             const float w = a.win[(size_t)ky * N + x0 + c];
             const bool masked = amp[(size_t)ky * N + x0 + c] < 0.f;
@@ -589,7 +589,6 @@ struct CorrSpecArgs {
     const float* amp;
     const float2* tw;
     const float* win;       // k_corr_window's table
-    int unit_scale;         // apply normalize_ft_shift (z *= |z|/|z|) to d and r first
 };
 
 template <int N>
@@ -612,11 +611,7 @@ __global__ __launch_bounds__(AuxGeo<N>::COL_THREADS) void k_corr_spec_cols(CorrS
     float2 v[V], v2[V];   // both products at once, as in ACOL_CORR
 #pragma unroll
     for (int q = 0; q < V; ++q) {
-        float2 dv = d[off + q * T * N], rv = r[off + q * T * N];
-        if (a.unit_scale) {
-            dv = unit_scaled(dv);
-            rv = unit_scaled(rv);
-        }
+        const float2 dv = d[off + q * T * N], rv = r[off + q * T * N];
         const float w = a.win[x0 + off + q * T * N];
         const bool masked = amp[off + q * T * N] < 0.f;
         v[q] = corr_product(dv, rv, -1.f, w, masked);

@@ -185,27 +185,18 @@ PhaseCut cut_raar(float r) {
 template <int N, int RV> int launch_row_v(spr_ctx* c, int mode, const RowArgs& a, int cnt, hipStream_t s) {
     using G = typename RowVariant<N, RV>::G;
     const dim3 grid((unsigned)((size_t)cnt * N / G::RW)), block(G::ROW_THREADS);
-    if constexpr (G::ROW_RECOMPUTE) {
-        if (mode == ROW_HIO || mode == ROW_RAAR || mode == ROW_ER) {
-            if (mode == ROW_HIO) hipLaunchKernelGGL((k_row_listed<N, ROW_HIO, RV>), grid, block, 0, s, a, cnt);
-            else if (mode == ROW_RAAR) hipLaunchKernelGGL((k_row_listed<N, ROW_RAAR, RV>), grid, block, 0, s, a, cnt);
-            else hipLaunchKernelGGL((k_row_listed<N, ROW_ER, RV>), grid, block, 0, s, a, cnt);
-            SPR_HIP(c, hipGetLastError());
-            return SPR_OK;
-        }
-    }
+    // The update on every row, or on the listed ones.
+    auto update = [&](auto m) {
+        constexpr int MODE = decltype(m)::value;
+        if constexpr (G::ROW_RECOMPUTE) hipLaunchKernelGGL((k_row_listed<N, MODE, RV>), grid, block, 0, s, a, cnt);
+        else hipLaunchKernelGGL((k_row<N, MODE, RV>), grid, block, 0, s, a);
+    };
     switch (mode) {
         case ROW_FWD: hipLaunchKernelGGL((k_row<N, ROW_FWD, RV>), grid, block, 0, s, a); break;
         case ROW_FINAL: hipLaunchKernelGGL((k_row<N, ROW_FINAL, RV>), grid, block, 0, s, a); break;
-        case ROW_HIO:
-            if constexpr (!G::ROW_RECOMPUTE) hipLaunchKernelGGL((k_row<N, ROW_HIO, RV>), grid, block, 0, s, a);
-            break;
-        case ROW_RAAR:
-            if constexpr (!G::ROW_RECOMPUTE) hipLaunchKernelGGL((k_row<N, ROW_RAAR, RV>), grid, block, 0, s, a);
-            break;
-        case ROW_ER:
-            if constexpr (!G::ROW_RECOMPUTE) hipLaunchKernelGGL((k_row<N, ROW_ER, RV>), grid, block, 0, s, a);
-            break;
+        case ROW_HIO: update(std::integral_constant<int, ROW_HIO>{}); break;
+        case ROW_RAAR: update(std::integral_constant<int, ROW_RAAR>{}); break;
+        case ROW_ER: update(std::integral_constant<int, ROW_ER>{}); break;
         case ROW_FWD_INPLACE: hipLaunchKernelGGL((k_row<N, ROW_FWD_INPLACE, RV>), grid, block, 0, s, a); break;
         case ROW_INV_INPLACE: hipLaunchKernelGGL((k_row<N, ROW_INV_INPLACE, RV>), grid, block, 0, s, a); break;
         default: return fail(c, SPR_ERR_ARG, "bad row mode");
@@ -256,7 +247,7 @@ template <int N, int CV>
 int launch_col_v(spr_ctx* c, int mode, float2* f, int cnt, hipStream_t s, int first) {
     using G = typename ColVariant<N, CV>::G;
     if (G::TW_GLOBAL && !c->twtab[CV]) return fail(c, SPR_ERR_STATE, "twiddle table missing");
-    const ColArgs a{f, c->amp, c->tw, c->amp_t, c->amp_of ? c->amp_of + first : nullptr, c->twtab[CV], f};
+    const ColArgs a{f, c->amp, c->tw, c->amp_t, c->amp_of ? c->amp_of + first : nullptr, c->twtab[CV]};
     const dim3 grid((unsigned)((size_t)cnt * (N / G::C))), block(G::COL_THREADS);
     switch (mode) {
         case COL_PROJ: hipLaunchKernelGGL((k_col<N, COL_PROJ, CV>), grid, block, 0, s, a); break;
@@ -691,9 +682,6 @@ int queue_symmetry(spr_ctx* c, float symmin, float symmax) {
     AuxColArgs ca = aux_col_args(c);
     SPR_TRY2(corr_window(c, symmin, symmax));
     ca.win = c->corrwin;
-    ca.unit_scale = 1;
-    ca.ref = nullptr;
-    ca.ref_index = nullptr;
     SPR_TRY2(col_aux(c, ACOL_CORR, ca, c->P));
     SPR_TRY2(fill_u64(c, c->keys, 0ull, 2 * (size_t)c->cap));
     SPR_TRY2(row_aux(c, AROW_CORR, a, c->P));
@@ -986,9 +974,8 @@ int pick_shifts(spr_ctx* c, const float* pdirect, const float* pflip, ShiftParam
 // Correlate spectra d_index[i] against r_index[i] in the window of corr_window,
 // pick the shifts and write them to shiftp (first index of the strict maximum,
 // direct vs twin).
-int correlate_and_pick(spr_ctx* c, const float2* spec, const int* d_index, const int* r_index, int unit_scale,
-                       const float* pdirect, const float* pflip, ShiftParam* shiftp,
-                       int items) {
+int correlate_and_pick(spr_ctx* c, const float2* spec, const int* d_index, const int* r_index,
+                       const float* pdirect, const float* pflip, ShiftParam* shiftp, int items) {
     CorrSpecArgs ca{};
     ca.spec = spec;
     ca.d_index = d_index;
@@ -996,7 +983,6 @@ int correlate_and_pick(spr_ctx* c, const float2* spec, const int* d_index, const
     ca.out1 = c->work;
     ca.out2 = c->work2;
     ca.win = c->corrwin;
-    ca.unit_scale = unit_scale;
     SPR_TRY2(corr_spec(c, ca, items));
     return pick_shifts(c, pdirect, pflip, shiftp, items);
 }
@@ -1930,7 +1916,6 @@ int spr_align(spr_ctx* c, const float* ref_rho, float minr, float maxr, const fl
     ca.f = c->work;
     ca.ref = spec;
     ca.win = c->corrwin;
-    ca.unit_scale = 1;
     SPR_TRY(col_aux(c, ACOL_CORR, ca, P));
     SPR_TRY(pick_shifts(c, ph, ph + P, sp, P));
     ReshiftArgs ra{};
@@ -2144,7 +2129,7 @@ int spr_crossover(spr_ctx* c, int nchild, const spr_cross_desc* desc, const int3
     if (with_avg) SPR_TRY(modulus_spectra(c, (const float2*)c->fieldbuf.p, nullptr, spec + (size_t)P * np, 1));
     // reshift_parent of p0, p2, p3 (and the average) against p1
     for (int r = 0; r < (with_avg ? 4 : 3); ++r) {
-        SPR_TRY(correlate_and_pick(c, spec, dlist(I_D, r), dlist(I_R, r), 0, dph + (size_t)r * 2 * K,
+        SPR_TRY(correlate_and_pick(c, spec, dlist(I_D, r), dlist(I_R, r), dph + (size_t)r * 2 * K,
                                    dph + (size_t)r * 2 * K + K, sp, K));
         ReshiftArgs ra{};
         ra.src = r < 3 ? c->rho : (const float2*)c->fieldbuf.p;

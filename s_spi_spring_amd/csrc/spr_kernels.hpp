@@ -728,7 +728,6 @@ struct ColArgs {
     const float* amp_t; // the amplitudes transposed, amp_t[x*N + y] = amp[y*N + x]
     const int* amp_of;  // field -> pattern (NULL: every field belongs to pattern 0)
     const float2* twtab;  // the plan's twiddle table in global memory (variants with TW_GLOBAL)
-    float2* out;          // output fields (= f: in place)
 };
 
 // Offset of the amplitude of field p (block-uniform: one scalar load).
@@ -792,7 +791,6 @@ __attribute__((amdgpu_waves_per_eu((ColVariant<N, CV>::G::COL_WAVES_PER_EU)))) v
     const int x0 = (strip % TILES) * C;
     // Block-uniform bases with 32-bit per-thread offsets (SGPR base addressing).
     float2* __restrict__ f = a.f + (size_t)p * N * N + x0;
-    float2* __restrict__ fo = a.out + (size_t)p * N * N + x0;
     const int off = t * N + c;
     float2 v[V];
 #pragma unroll
@@ -839,7 +837,7 @@ __attribute__((amdgpu_waves_per_eu((ColVariant<N, CV>::G::COL_WAVES_PER_EU)))) v
         if constexpr (MODE == COL_PROJ || MODE == COL_INV) fft_line_p<PL, -1>(v, acc, tw, t);
     }
 #pragma unroll
-    for (int q = 0; q < V; ++q) st_stream(fo + off + q * T * N, v[q]);
+    for (int q = 0; q < V; ++q) st_stream(f + off + q * T * N, v[q]);
 }
 
 // ---------------------------------------------------------------------------
