@@ -324,11 +324,6 @@ int spr_stream(spr_ctx* ctx, void** stream);
  *   of that size created later in the process; col_ms / row_ms (NULL or one
  *   entry per variant) receive the mean iteration durations in ms.
  * spr_set_variants / spr_get_variants: one handle's pair.
- * spr_get_plain_variant: the column variant of the handle's projection passes
- *   outside an iteration with a recomputed state (the trailing projection,
- *   shrink-wrap). On a handle with the compiled choice it may be another
- *   variant of the same radix plan than spr_get_variants' column; variants set
- *   by the caller or by spr_autotune run as they are in every pass.
  * spr_default_variants / spr_set_default_variants: the pair new handles of
  *   size n start with (initially the table compiled from the last autotuning
  *   run on the target GPU, spr_tuned.hpp).
@@ -362,7 +357,6 @@ int spr_get_fused(spr_ctx* ctx, int* mode, int* active);
 int spr_autotune(spr_ctx* ctx, int reps, float* col_ms, float* row_ms);
 int spr_set_variants(spr_ctx* ctx, int col, int row);
 int spr_get_variants(spr_ctx* ctx, int* col, int* row);
-int spr_get_plain_variant(spr_ctx* ctx, int* col);
 int spr_default_variants(int n, int* col, int* row);
 int spr_set_default_variants(int n, int col, int row);
 

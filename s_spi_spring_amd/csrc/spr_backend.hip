@@ -67,7 +67,6 @@ struct spr_ctx {
     float* amp_t = nullptr;       // amp transposed (read along columns by the column pass)
     int npat = 1;                 // patterns sharing this handle (one amplitude each)
     int colvar = 0, rowvar = 0;   // variants of the column and row iteration passes
-    bool exact = false;           // chosen by the caller or the autotuner: the plain projection runs colvar itself
     const float2* twtab[MAX_VARIANTS] = {};  // twiddle tables of the column variants, behind tw
     size_t chunk_bytes = 0;       // iteration blocks run in chunks of this working set (0: whole population)
     int fused = -1;               // on-chip iteration blocks (N <= 128): -1 by population size, 0 never, 1 always
@@ -341,27 +340,15 @@ template <int N, int CV = 0> void append_twtabs(const std::vector<float2>& root,
     }
 }
 
-// Column variant of the plain projection: the handle's, or, where the handle runs
-// the compiled choice, the one plain_variant names beside it.
-template <int N, int CV = 0> int plain_colvar(const spr_ctx* c) {
-    if (c->exact) return c->colvar;
-    if constexpr (CV < MAX_VARIANTS) return c->colvar == CV ? plain_variant<N, CV>() : plain_colvar<N, CV + 1>(c);
-    return c->colvar;
-}
 template <int N, int CV = 0> int launch_col(spr_ctx* c, int mode, float2* f, int cnt, hipStream_t s, int first) {
     if (mode != COL_PROJ) return launch_col_v<N, 0>(c, mode, f, cnt, s, first);
     if constexpr (CV < MAX_VARIANTS) {
         if constexpr (ColVariant<N, CV>::valid)
-            if (plain_colvar<N>(c) == CV) return launch_col_v<N, CV>(c, mode, f, cnt, s, first);
+            if (c->colvar == CV) return launch_col_v<N, CV>(c, mode, f, cnt, s, first);
         return launch_col<N, CV + 1>(c, mode, f, cnt, s, first);
     } else {
         return fail(c, SPR_ERR_ARG, "bad column variant");
     }
-}
-
-template <int N> int plain_colvar_n(spr_ctx* c, int* col) {
-    *col = plain_colvar<N>(c);
-    return SPR_OK;
 }
 
 // Grid sizes with compiled kernels (RadixPlan in spr_fft.hpp).
@@ -786,10 +773,14 @@ int queue_iterate_lanes(spr_ctx* c, int mode, int niter, const RowArgs& a0) {
 }
 
 // Individuals per chunk of an iteration block: the population split into the
-// fewest equal chunks whose densities, fields and supports (17 bytes per pixel;
-// with the recomputed state the iterations touch the two field buffers and the
-// support bits instead, about as much) fit in c->chunk_bytes (at least one
-// individual per chunk).
+// fewest equal chunks whose densities, fields and supports (17 bytes per pixel) fit
+// in c->chunk_bytes (at least one individual per chunk). With the recomputed state
+// the iterations touch 8 + 8 h bytes per pixel instead, h the listed fraction, but the
+// same 300 MB is the best or nearly the best cap for both a quarter of the rows and
+// all of them; us per RAAR iteration, whole / 450 / 300 / 200 MB: 512^2 x 256, h = 1/4
+// 394 / 388 / 338 / 344, h = 1 620 / 581 / 501 / 497; 768^2 x 56 262 / 214 / 214 / 236,
+// 357 / 305 / 307 / 314; 1024^2 x 64 417 / 389 / 386 / 427, 656 / 660 / 584 / 594;
+// 384^2 x 256 230 / 187 / 204 / 214, 382 / 335 / 295 / 314.
 int chunk_individuals(const spr_ctx* c) {
     if (c->chunk_bytes == 0 || c->P <= 1) return std::max(c->P, 1);
     const size_t per = (size_t)17 * c->n * c->n;
@@ -1017,7 +1008,7 @@ template <int N, int CV> constexpr bool same_plan_variant() {
 template <int N, int CV = 0> int launch_col_grad(spr_ctx* c, const LossArgs& a, int items) {
     if constexpr (CV < MAX_VARIANTS) {
         if constexpr (same_plan_variant<N, CV>())
-            if (plain_colvar<N>(c) == CV) return launch_col_loss_v<N, CV>(c, a, items, false);
+            if (c->colvar == CV) return launch_col_loss_v<N, CV>(c, a, items, false);
         return launch_col_grad<N, CV + 1>(c, a, items);
     }
     return launch_col_loss_v<N, 0>(c, a, items, false);
@@ -1028,8 +1019,8 @@ template <int N> int launch_col_loss(spr_ctx* c, const LossArgs& a, int items, b
 }
 // The loss pass with one loss partial per workgroup (n / cols_per_wg(n) per
 // field) in the default geometry, and the refinement steps' gradient pass
-// without partials, in the handle's column variant (the plain projection's) when
-// that variant holds the default radix plan (the same gradients as spr_loss_grad,
+// without partials, in the handle's column variant when that
+// variant holds the default radix plan (the same gradients as spr_loss_grad,
 // bit for bit), else in the default geometry too (at 1024^2 the radix-16 variants
 // measured no faster for this pass: 0.577 against 0.575 ms per refinement step).
 int col_loss(spr_ctx* c, const LossArgs& a, int items) { SPR_DISPATCH_N(c, launch_col_loss, c, a, items, true); }
@@ -1154,7 +1145,6 @@ int final_loss(spr_ctx* c, int kind, float eps, double* loss) {
 // ---------------------------------------------------------------------------
 struct VariantPair {
     int col = 0, row = 0;
-    bool exact = false;    // chosen at run time, not from the compiled table
 };
 std::mutex g_variant_mu;
 std::map<int, VariantPair> g_variant;   // sizes whose default differs from the compiled table
@@ -1245,7 +1235,7 @@ int autotune(spr_ctx* c, int reps, float* col_ms, float* row_ms) {
     RowArgs ra = row_args(c);
     ra.beta = 0.87f;
     ra.pc = cut_raar(0.f);
-    const VariantPair keep{c->colvar, c->rowvar, c->exact};
+    const VariantPair keep{c->colvar, c->rowvar};
     hipEvent_t e0 = nullptr, e1 = nullptr;
     SPR_HIP(c, hipEventCreate(&e0));
     if (hipEventCreate(&e1) != hipSuccess) {
@@ -1265,8 +1255,6 @@ int autotune(spr_ctx* c, int reps, float* col_ms, float* row_ms) {
     float tc[MAX_VARIANTS] = {}, tr[MAX_VARIANTS] = {};
     int rc = SPR_OK;
     VariantPair best;
-    best.exact = true;
-    c->exact = true;   // every variant is timed as itself
     for (int v = 0; v < nc && rc == SPR_OK; ++v) {
         c->colvar = v;
         rc = time_iteration(c, ra, reps, e0, e1, &tc[v]);
@@ -1285,7 +1273,6 @@ int autotune(spr_ctx* c, int reps, float* col_ms, float* row_ms) {
     if (rc != SPR_OK) {
         c->colvar = keep.col;
         c->rowvar = keep.row;
-        c->exact = keep.exact;
         return rc;
     }
     c->colvar = best.col;
@@ -1435,7 +1422,6 @@ static int create_context(spr_ctx** out, int n, int capacity, int npat, const fl
         const VariantPair v = default_variants(n);
         c->colvar = v.col;
         c->rowvar = v.row;
-        c->exact = v.exact;
     }
     const size_t np = (size_t)n * n;
     auto cleanup_fail = [&](const char* what, hipError_t e) {
@@ -2365,7 +2351,7 @@ int spr_set_default_variants(int n, int col, int row) {
     if (variant_counts(n, &nc, &nr) != SPR_OK) return fail(nullptr, SPR_ERR_ARG, "unsupported grid size");
     if (col < 0 || col >= nc || row < 0 || row >= nr) return fail(nullptr, SPR_ERR_ARG, "variant out of range");
     std::lock_guard<std::mutex> lk(g_variant_mu);
-    g_variant[n] = VariantPair{col, row, true};
+    g_variant[n] = VariantPair{col, row};
     return SPR_OK;
 }
 
@@ -2377,7 +2363,6 @@ int spr_set_variants(spr_ctx* c, int col, int row) {
     SPR_HIP(c, hipStreamSynchronize(c->stream));
     c->colvar = col;
     c->rowvar = row;
-    c->exact = true;
     return SPR_OK;
 }
 
@@ -2386,11 +2371,6 @@ int spr_get_variants(spr_ctx* c, int* col, int* row) {
     if (col) *col = c->colvar;
     if (row) *row = c->rowvar;
     return SPR_OK;
-}
-
-int spr_get_plain_variant(spr_ctx* c, int* col) {
-    if (!c || !col) return fail(c, SPR_ERR_ARG, "NULL argument");
-    SPR_DISPATCH_N(c, plain_colvar_n, c, col);
 }
 
 int spr_set_chunk(spr_ctx* c, long long bytes) {

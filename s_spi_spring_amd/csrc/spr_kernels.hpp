@@ -29,9 +29,10 @@
 //                                                                 24.125 h B/px
 // so HIO/RAAR move 48.125 or 16 + 24.125 h B/px per individual-iteration (the second
 // form saves the state's round trip for one more row transform in HIO and none
-// in RAAR); ER, which needs no rho_n, moves 32.125 B/px in both. proj is the
-// work2 buffer. (The support packing reads 1 and writes 0.125 B/px once per
-// block.)
+// in RAAR); ER, which needs no rho_n, moves 32.125 B/px in the first form and, its
+// other rows being zero, 32.125 h in the second. proj is the work2 buffer. (The
+// support packing reads 1 and writes 0.125 B/px once per block.) Where nearly every
+// row meets the support, all are listed (h = 1) and the column pass updates none.
 #pragma once
 
 #include <cstdint>
@@ -160,10 +161,11 @@ SPR_COL_VARIANT(1024, 7, RadixPlan<1024>, 8, 256, -1, 1, 1)
 SPR_COL_VARIANT(2048, 1, RadixPlan<2048>, 4, 256, -1, 0, 1)
 SPR_COL_VARIANT(2048, 2, Plan<2048, 16, 16, 8, 16>, 8, 256, -1, 0, 1)
 // (plan, columns, -, -, -, -, -, spare tile row every 2^k rows, waves per SIMD):
-// tiles without the bank conflicts of the padded layouts. Their address
-// arithmetic takes registers, which k_col_step lacks: with 80 (512^2, 8 columns)
-// it spills and the iteration takes 0.080 ms against 0.077 in the padded tile;
-// the plain projection pass is ahead in them (52 against 60 us).
+// tiles without the bank conflicts of the padded layouts. us per launch of the plain
+// projection, padded / skewed: 512^2 x 64, 8 columns 62.8 / 50.8; 768^2 x 28, 4 columns
+// 84.0 / 73.6; per RAAR and ER iteration with a quarter of the rows listed 86.5 and
+// 67.3 / 85.8 and 62.1; 109.8 and 92.8 / 104.3 and 84.1. At 1024^2 (8 columns in 128
+// registers) their address arithmetic makes k_col_step spill: 116.4 against 98.6.
 SPR_COL_VARIANT(512, 6, RadixPlan<512>, 8, 256, -1, 0, 0, 3, 3)
 SPR_COL_VARIANT(512, 7, RadixPlan<512>, 4, 256, -1, 0, 0, 3, 2, 5)
 SPR_COL_VARIANT(768, 1, RadixPlan<768>, 4, 256, -1, 1, 0, 3, 2, 3)
@@ -204,19 +206,6 @@ SPR_ROW_VARIANT(2048, 4, RadixPlan<2048>, 0, 256, -1, 1, 0, 4, 0, 0, 1)
 SPR_ROW_VARIANT(2048, 5, Plan<2048, 16, 16, 8, 16>, 0, 256, -1, 1, 0, 4, 0, 0, 1)
 #undef SPR_COL_VARIANT
 #undef SPR_ROW_VARIANT
-
-// The column variant of the plain projection (k_col) and of the refinement's gradient
-// pass where CV is the compiled choice of the step pass: the same plan in the layout
-// that k_col runs best in, where that differs by more than its 5 % of noise. us per
-// launch, CV / here: 512^2 x 64 62.8 / 50.8, 768^2 x 28 84.0 / 69.9; 256^2 x 128
-// 25.8 in variant 2, 26.0 in variant 1; 384^2 x 64 37.8, the others from 38.8;
-// 1024^2 x 16 67.7 in variant 6, 67.9 in variant 4; 2048^2 x 4 99.5, the others from
-// 100.9.
-template <int N, int CV> constexpr int plain_variant() {
-    if constexpr (N == 512 && CV == 1) return 6;
-    else if constexpr (N == 768 && CV == 2) return 7;
-    else return CV;
-}
 
 constexpr int MAX_VARIANTS = 8;
 template <int N> constexpr int col_variants() {
@@ -900,16 +889,12 @@ __device__ __forceinline__ int row_offset(int voff, uint32_t off_rows, int q) {
     return voff | (int)((off_rows << (31 - q)) & 0x80000000u);
 }
 
-// STEP_LIN of a field whose every row is listed: the plain projection, into proj,
-// in the tile layout that is best for it (plain_variant), which the registers of the
-// other path do not leave room for.
+// STEP_LIN of a field whose every row is listed: the plain projection, into proj.
 template <int N, class G>
 __device__ __forceinline__ void step_every_row(const StepArgs& a, float2* lds, const float2* tw, int p, int t, int c, int x0) {
     using PL = typename G::PL;
     constexpr int V = G::V, T = G::T, C = G::C;
-    constexpr int SKEW = G::COL_SKEW > 0 ? G::COL_SKEW : (N == 512 || N == 768) && G::CS == C + 1 ? log2i(C) : 0;
-    using Acc = std::conditional_t<(SKEW > 0), ColAccSkew<C, (SKEW > 0 ? SKEW : 1)>, ColAcc<G::CS>>;
-    static_assert(SKEW == 0 || (N + (N >> SKEW)) * C <= G::COL_TILE, "the skewed tile fits in the padded one");
+    using Acc = std::conditional_t<(G::COL_SKEW > 0), ColAccSkew<C, (G::COL_SKEW > 0 ? G::COL_SKEW : 1)>, ColAcc<G::CS>>;
     const float2* __restrict__ f = a.f + (size_t)p * N * N + x0;
     const float* __restrict__ amp = a.amp + amp_offset<N>(a.amp_of, p) + x0;
     float2* __restrict__ proj = a.proj + (size_t)p * N * N + x0;

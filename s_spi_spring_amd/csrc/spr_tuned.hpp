@@ -11,10 +11,10 @@ struct TunedVariants {
 constexpr TunedVariants kTuned[] = {
     {256, 2, 3},
     {384, 1, 3},
-    {512, 1, 3},
-    {768, 2, 4},
-    {1024, 6, 6},
-    {2048, 2, 5},
+    {512, 6, 3},
+    {768, 6, 4},
+    {1024, 3, 6},
+    {2048, 2, 4},
 };
 
 }  // namespace spr

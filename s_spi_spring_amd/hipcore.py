@@ -82,7 +82,6 @@ SIGNATURES = {
     "spr_row_variant_info": (_I, [_I, _I, ctypes.POINTER(_I)]),
     "spr_set_variants": (_I, [_VP, _I, _I]),
     "spr_get_variants": (_I, [_VP, ctypes.POINTER(_I), ctypes.POINTER(_I)]),
-    "spr_get_plain_variant": (_I, [_VP, ctypes.POINTER(_I)]),
     "spr_default_variants": (_I, [_I, ctypes.POINTER(_I), ctypes.POINTER(_I)]),
     "spr_set_default_variants": (_I, [_I, _I, _I]),
 }
@@ -418,12 +417,6 @@ class Backend:
         c, r = ctypes.c_int(), ctypes.c_int()
         self._check(self.lib.spr_get_variants(self.h, ctypes.byref(c), ctypes.byref(r)))
         return c.value, r.value
-
-    def plain_variant(self):
-        """Column variant of the projection passes outside an iteration with a recomputed state."""
-        c = ctypes.c_int()
-        self._check(self.lib.spr_get_plain_variant(self.h, ctypes.byref(c)))
-        return c.value
 
     def set_variants(self, col, row):
         self._check(self.lib.spr_set_variants(self.h, int(col), int(row)))

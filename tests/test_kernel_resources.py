@@ -62,3 +62,29 @@ def test_loss_passes_of_1024_run_two_workgroups_on_a_cu(kernels):
         scratch = k[".private_segment_fixed_size"]
         assert k[".vgpr_count"] <= 64 and scratch <= (32 if "ELb1E" in name else 0), (name, k[".vgpr_count"], scratch)
         assert 2 * k[".group_segment_fixed_size"] <= 160 * 1024, name
+
+
+SIZES = [64, 128, 256, 384, 512, 768, 1024, 2048]
+
+
+def test_every_column_variant_has_its_own_passes(kernels):
+    """A variant that a caller sets runs its own kernels, not another variant's in its place."""
+    for n in SIZES:
+        steps = any(hipcore.row_variant_recomputes_state(n, r) for r in range(hipcore.variant_counts(n)[1]))
+        for v in range(hipcore.variant_counts(n)[0]):
+            named(kernels, rf"5k_colILi{n}ELi0ELi{v}EE")
+            for mode in range(3 if steps else 0):
+                named(kernels, rf"10k_col_stepILi{n}ELi{mode}ELi{v}EE")
+
+
+def test_compiled_choice_of_the_iteration_passes_spills_nothing(kernels):
+    for n in SIZES[2:]:
+        col, row = hipcore.default_variants(n)
+        for name, k in named(kernels, rf"(10k_col_stepILi{n}ELi[01]ELi{col}EE|12k_row_listedILi{n}ELi\dELi{row}EE)").items():
+            # 2048^2: 32 values of 8 bytes, field and state, in 128 registers
+            assert k[".private_segment_fixed_size"] <= (64 if n == 2048 else 0), (name, k[".private_segment_fixed_size"])
+
+
+def test_on_chip_blocks_spill_little(kernels):
+    for name, k in named(kernels, r"k_iter_fusedILi(64|128)").items():
+        assert k[".private_segment_fixed_size"] <= 16, (name, k[".private_segment_fixed_size"])
