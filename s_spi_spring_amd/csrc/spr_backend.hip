@@ -203,6 +203,26 @@ template <int N, int RV> int launch_row_v(spr_ctx* c, int mode, const RowArgs& a
     SPR_HIP(c, hipGetLastError());
     return SPR_OK;
 }
+// The first row pass of a block with the row lists of its individuals.
+template <int N, int RV = 0>
+int launch_row_first(spr_ctx* c, const RowArgs& a, const SupportPlan& plan, int cnt, hipStream_t s) {
+    if constexpr (RV < MAX_VARIANTS) {
+        if constexpr (RowVariant<N, RV>::valid) {
+            using G = typename RowVariant<N, RV>::G;
+            if constexpr (G::ROW_RECOMPUTE) {
+                if (c->rowvar == RV) {
+                    hipLaunchKernelGGL((k_row_first<N, RV>), dim3((unsigned)((size_t)cnt * N / G::RW)),
+                                       dim3(G::ROW_THREADS), 0, s, (const float2*)a.rho, a.work, a.tw, plan);
+                    SPR_HIP(c, hipGetLastError());
+                    return SPR_OK;
+                }
+            }
+        }
+        return launch_row_first<N, RV + 1>(c, a, plan, cnt, s);
+    } else {
+        return fail(c, SPR_ERR_ARG, "no row lists with this row variant");
+    }
+}
 template <int N> int launch_row(spr_ctx* c, int mode, const RowArgs& a, int cnt, hipStream_t s) {
     switch (c->rowvar) {
         case 0: return launch_row_v<N, 0>(c, mode, a, cnt, s);
@@ -369,6 +389,9 @@ template <int N, int CV = 0> int launch_col(spr_ctx* c, int mode, float2* f, int
 
 int row_n(spr_ctx* c, int mode, const RowArgs& a, int cnt, hipStream_t s) {
     SPR_DISPATCH_N(c, launch_row, c, mode, a, cnt, s);
+}
+int row_first_n(spr_ctx* c, const RowArgs& a, const SupportPlan& plan, int cnt, hipStream_t s) {
+    SPR_DISPATCH_N(c, launch_row_first, c, a, plan, cnt, s);
 }
 // Column pass over fields f[0, cnt), the individuals [first, first + cnt), in place.
 int col_n(spr_ctx* c, int mode, float2* f, int cnt, hipStream_t s, int first = 0) {
@@ -708,13 +731,20 @@ SupportPlan support_plan(const spr_ctx* c, int first) {
                        c->colmask + f * lines, c->rowflags + f * (c->n / 32), c->n, lines};
 }
 // The support bits of all resident individuals, and the flags that the first row pass
-// makes row lists and column masks from.
+// (first_rows) makes row lists and column masks from.
 int pack_support(spr_ctx* c, hipStream_t s) {
     if (c->P <= 0) return SPR_OK;
     hipLaunchKernelGGL(k_pack_support, dim3((unsigned)(c->n / 32 * c->P)), dim3(pack_threads(c->n)), 0, s,
                        support_plan(c, 0));
     SPR_HIP(c, hipGetLastError());
     return SPR_OK;
+}
+
+// The first row pass of a block over individuals [first, first + cnt), whose fields `a`
+// points to; a block without iterations reads no row lists.
+int first_rows(spr_ctx* c, const RowArgs& a, bool rs, int niter, int cnt, hipStream_t s, int first) {
+    if (rs && niter > 0) return row_first_n(c, a, support_plan(c, first), cnt, s);
+    return row_n(c, ROW_FWD, a, cnt, s);
 }
 
 // The projection pass of iteration i of a block (i = niter: the trailing one) over
@@ -742,13 +772,8 @@ int queue_iterate_lanes(spr_ctx* c, int mode, int niter, const RowArgs& a0) {
     const int h = (c->P + 1) / 2, h2 = c->P - h;
     const size_t off = (size_t)h * c->n * c->n;
     const bool rs = row_recomputes(c->n, c->rowvar);
-    RowArgs a = a0;
-    if (niter > 0) {
-        SPR_TRY(pack_support(c, c->stream));
-        a.plan = support_plan(c, 0);
-    }
+    const RowArgs a = a0;
     RowArgs b = a;
-    if (niter > 0) b.plan = support_plan(c, h);
     b.rho += off;
     b.work += off;
     b.supp += off;
@@ -757,10 +782,11 @@ int queue_iterate_lanes(spr_ctx* c, int mode, int niter, const RowArgs& a0) {
     b.rowlist += (size_t)h * c->n;
     b.proj += off;
     hipStream_t s1 = c->stream, s2 = c->lane2;
-    SPR_TRY(row_n(c, ROW_FWD, a, h, s1));
+    if (niter > 0) SPR_TRY(pack_support(c, s1));
+    SPR_TRY(first_rows(c, a, rs, niter, h, s1, 0));
     SPR_HIP(c, hipEventRecord(c->ev_fork, s1));
     SPR_HIP(c, hipStreamWaitEvent(s2, c->ev_fork, 0));
-    SPR_TRY(row_n(c, ROW_FWD, b, h2, s2));
+    SPR_TRY(first_rows(c, b, rs, niter, h2, s2, h));
     for (int i = 0; i <= niter; ++i) {
         SPR_TRY(project(c, mode, a, rs, i, niter, h, s1, 0));
         SPR_TRY(project(c, mode, b, rs, i, niter, h2, s2, h));
@@ -805,7 +831,6 @@ int queue_iterate_block(spr_ctx* c, int mode, int niter, const RowArgs& a0) {
     for (int first = 0; first < c->P; first += chunk) {
         const int cnt = std::min(chunk, c->P - first);
         RowArgs a = a0;
-        if (niter > 0) a.plan = support_plan(c, first);
         a.rho += first * np;
         a.work += first * np;
         a.supp += first * np;
@@ -813,7 +838,9 @@ int queue_iterate_block(spr_ctx* c, int mode, int niter, const RowArgs& a0) {
         a.rowcnt += first;
         a.rowlist += (size_t)first * c->n;
         a.proj += first * np;
-        SPR_TRY(row(c, ROW_FWD, a, cnt));
+        SPR_TRY(timing_begin(c, SPR_KIND_ROW_OTHER));
+        SPR_TRY(first_rows(c, a, rs, niter, cnt, c->stream, first));
+        SPR_TRY(timing_end(c));
         for (int i = 0; i <= niter; ++i) {
             SPR_TRY(timing_begin(c, SPR_KIND_COL_PROJ));
             SPR_TRY(project(c, mode, a, rs, i, niter, cnt, c->stream, first));
@@ -1196,8 +1223,7 @@ int time_iteration(spr_ctx* c, const RowArgs& ra0, int reps, hipEvent_t e0, hipE
     RowArgs ra = ra0;
     const bool rs = row_recomputes(c->n, c->rowvar);
     SPR_TRY(pack_support(c, c->stream));
-    ra.plan = support_plan(c, 0);   // the column masks follow the column variant
-    SPR_TRY(row_n(c, ROW_FWD, ra, c->P, c->stream));
+    SPR_TRY(first_rows(c, ra, rs, 1, c->P, c->stream, 0));   // the column masks follow the column variant
     if (!rs) {
         const int np = c->n * c->n;
         hipLaunchKernelGGL(k_copy_fields, dim3((np + 255) / 256, c->P), dim3(256), 0, c->stream, (const float2*)c->rho,

@@ -424,7 +424,6 @@ struct RowArgs {
     // their number and, ascending, their indices.
     const int* rowcnt;       // [fields]
     const uint16_t* rowlist; // [fields][N]
-    SupportPlan plan;        // ROW_FWD: made for each field where plan.lines > 0
 };
 
 // Support bit of pixel i of a field: bit i&31 of word i>>5 (N*N and the
@@ -542,13 +541,6 @@ __global__ __launch_bounds__((RowVariant<N, RV>::G::ROW_THREADS)) void k_row(Row
         float2* dst = (MODE == ROW_FWD) ? work : rho;
 #pragma unroll
         for (int q = 0; q < V; ++q) dst[off + q * T] = v[q];
-        if constexpr (MODE == ROW_FWD && G::ROW_RECOMPUTE) {
-            constexpr int GROUPS = N / G::RW;   // workgroups per field
-            if (a.plan.lines > 0 && blockIdx.x % GROUPS == 0) {
-                __syncthreads();
-                row_plan<N, G::ROW_THREADS>(a.plan, blockIdx.x / GROUPS, lds);
-            }
-        }
     } else if constexpr (MODE == ROW_FINAL || MODE == ROW_INV_INPLACE) {
         const float2* src = (MODE == ROW_FINAL) ? work : rho;
 #pragma unroll
@@ -597,6 +589,40 @@ __global__ __launch_bounds__((RowVariant<N, RV>::G::ROW_THREADS)) void k_row(Row
         fft_line_p<PL, +1, WV>(v, acc, tw, t);
 #pragma unroll
         for (int q = 0; q < V; ++q) st_stream(work + off + q * T, v[q]);
+    }
+}
+
+// The first row pass of a block that recomputes rho_n: work <- rowFFT+(rho), and the
+// fields' row lists. (A kernel of its own: the plan's pointers in RowArgs would go with
+// every launch, which for one individual costs 0.4 us each.)
+template <int N, int RV>
+__global__ __launch_bounds__((RowVariant<N, RV>::G::ROW_THREADS)) void k_row_first(const float2* __restrict__ rho,
+                                                                                   float2* __restrict__ work,
+                                                                                   const float2* __restrict__ roots,
+                                                                                   SupportPlan plan) {
+    using G = typename RowVariant<N, RV>::G;
+    using PL = typename G::PL;
+    constexpr int V = G::V, T = G::T;
+    constexpr bool WV = T <= 64;   // every row inside one wavefront: no workgroup barriers
+    __shared__ float2 tw[TwTableP<PL>::SIZE];
+    __shared__ float2 lds[G::RW * G::RS];
+    const int tid = threadIdx.x;
+    const int t = tid % T;
+    const int rl = tid / T;
+    tw_fill_p<PL>(tw, roots, tid, G::ROW_THREADS);
+    const size_t blk = (size_t)blockIdx.x * G::RW * N;
+    const int off = rl * N + t;
+    float2 v[V];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < V; ++r) v[r] = rho[blk + off + r * T];
+    fft_line_p<PL, +1, WV>(v, RowAccT<G::ROW_PAD_SHIFT>{lds + rl * G::RS}, tw, t);
+#pragma unroll
+    for (int q = 0; q < V; ++q) work[blk + off + q * T] = v[q];
+    constexpr int GROUPS = N / G::RW;   // workgroups per field
+    if (blockIdx.x % GROUPS == 0) {
+        __syncthreads();
+        row_plan<N, G::ROW_THREADS>(plan, blockIdx.x / GROUPS, lds);
     }
 }
 
